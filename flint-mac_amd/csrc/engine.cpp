@@ -384,17 +384,19 @@ void check_tokens(int n_tok, const char *name) {
 void proj_gemm(const MatvecSeg *seg, int n_seg, int N, int K, const float *x, long long x_stride, const float *norm_w,
                float eps, int T, float *y, long long y_stride, int add, const WeightPlanes *pl, hipStream_t stream,
                bool build_only = false) {
+    const IntForm form = gemm_int_form(seg, n_seg);
+    // short batches in the integer form read the GGUF rows themselves: no weight planes
+    const bool raw = form.sub && !build_only && T <= (pl ? GEMM_RAW_TOKENS_KEPT : GEMM_RAW_TOKENS);
     const int T_pass = build_only ? 0 : std::min(T, GEMM_PASS_TOKENS);
     const int T_pad = (T_pass + GEMM_TILE - 1) / GEMM_TILE * GEMM_TILE;
-    const size_t wbytes = pl ? 0 : (size_t)N * K * sizeof(_Float16), xbytes = (size_t)T_pad * K * sizeof(_Float16);
+    const size_t wbytes = pl || raw ? 0 : (size_t)N * K * sizeof(_Float16), xbytes = (size_t)T_pad * K * sizeof(_Float16);
     size_t off = 0;
     auto take = [&](size_t b) {
         const size_t o = off;
         off += (b + 255) / 256 * 256;
         return o;
     };
-    const size_t o_wh = take(wbytes), o_wl = take(wbytes), o_f = take(pl ? 0 : (size_t)N * sizeof(int));
-    const IntForm form = gemm_int_form(seg, n_seg);
+    const size_t o_wh = take(wbytes), o_wl = take(wbytes), o_f = take(pl || raw ? 0 : (size_t)N * sizeof(int));
     const size_t o_xh = take(xbytes), o_xl = take(xbytes), o_e = take((size_t)T_pad * sizeof(int));
     const size_t o_xs = take(form.min ? (size_t)T_pad * (K / 32) * sizeof(float) : 0);
     char *ws = off ? (char *)scratch().gemm.get(off) : nullptr;
@@ -421,6 +423,7 @@ void proj_gemm(const MatvecSeg *seg, int n_seg, int N, int K, const float *x, lo
     GemmParams G{};
     G.wh = W.wh, G.wl = W.wl, G.fexp = W.fexp, G.xh = X.xh, G.xl = X.xl, G.eexp = X.eexp;
     G.isub = W.isub, G.imin = W.imin, G.wd = W.wd, G.wm = W.wm, G.xs = X.xs;
+    G.raw = raw;
     G.add = add;
     G.N = N;
     G.K = K;
@@ -435,12 +438,13 @@ void proj_gemm(const MatvecSeg *seg, int n_seg, int N, int K, const float *x, lo
         X.x = x + (size_t)t0 * x_stride;
         X.x_stride = x_stride;
         X.T = n;
-        X.T_pad = (n + GEMM_TILE - 1) / GEMM_TILE * GEMM_TILE;
+        const int tile = raw ? GEMM_RAW_TILE : GEMM_TILE;
+        X.T_pad = (n + tile - 1) / tile * tile;
         G.y = y + (size_t)t0 * y_stride;
         G.y_stride = y_stride;
         G.T = n;
         // the weight planes are built once, in the first pass, unless the caller keeps them
-        check(launch_proj_gemm(W, X, G, !pl && t0 == 0, stream), "projection GEMM launch");
+        check(launch_proj_gemm(W, X, G, !pl && !raw && t0 == 0, stream), "projection GEMM launch");
     }
 }
 

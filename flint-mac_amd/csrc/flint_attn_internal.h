@@ -163,7 +163,20 @@ struct GemmParams {
     float *y;              // [T] rows of y_stride floats (16-byte aligned, stride a multiple of 4)
     long long y_stride;
     int add, N, K, T;
+    int raw;               // the integer form straight from the GGUF rows (no weight planes)
 };
+constexpr int GEMM_RAW_TILE = 32;    // tokens and rows per gemm_raw workgroup
+// Batches of the integer form up to these sizes take gemm_raw. Stage-level calls, q/k/v + o in q8_0: 16, 128,
+// 256, 384, 448 and 512 tokens 26.7, 37.9, 59, 85, 103 and 112 us against 142-145 us for the weight planes'
+// build and 128-token tiles (99-110 us with 64-token tiles and the faster build): the lines cross at 480, since
+// gemm_raw's 32 x 32 tiles read x and the rows once each. With the planes kept (no build), 49 blocks: 256, 320 and 384
+// tokens 4.15, 5.12 and 5.53 ms against 5.10, 5.19 and 5.30.
+constexpr int GEMM_RAW_TOKENS = 480, GEMM_RAW_TOKENS_KEPT = 320;
+// Batches up to this size take gemm_int's 64-token tiles, whose smaller workgroups fill the GPU sooner and hold
+// four stages. q/k/v + o in q8_0 (trace medians): 600 tokens 39 + 48 us against 47 + 80 with 128-token tiles, 1024
+// 61 + 52 against 62 + 84, 2048 110 + 86 against 116 + 105; at 4000 the larger tile reads less: 194 + 152 us.
+constexpr int GEMM_INT_64 = 2048;
+constexpr int GEMM_SEG = 512;         // the integer form sums K in segments of this many elements, then the segments
 constexpr int GEMM_TILE = 128;       // tokens and rows per gemm3 workgroup
 constexpr int GEMM_MIN_TOKENS = 16;  // batches from this size take the GEMM
 constexpr int GEMM_PASS_TOKENS = 8192;  // tokens per GEMM pass (a multiple of GEMM_TILE): bounds the workspace

@@ -264,6 +264,36 @@ def test_projection_rows_gemm_1000_tokens(cuda):
     _gemm_case(cuda, np.random.default_rng(61), ("q8_0", "q6_K", "q5_K"), "q8_0", 1000)
 
 
+@pytest.mark.parametrize("types,wo_type", [(("q8_0",) * 3, "q8_0"), (("q5_K",) * 3, "q5_K"), (("q5_K", "q8_0", "q6_K"), "q6_K"),
+                                           (("iq4_xs",) * 3, "iq4_xs"), (("f16", "bf16", "q5_K"), "f16"),
+                                           (("bf16", "iq4_xs", "q6_K"), "bf16")])
+def test_projection_rows_short_batches(cuda, types, wo_type):
+    """Short batches (the GEMM that reads the GGUF rows itself) at the edges of its tiles and range: 17
+    tokens within the oracle's bound; and, for 16, 17, 32, 33, 63, 480 and 481 tokens, every row has the bits
+    that a 600-token batch (the GEMM on weight planes) gives the same token."""
+    import torch
+    rng = np.random.default_rng(71)
+    _gemm_case(cuda, rng, types, wo_type, 17)
+    E, T = fa.N_EMBD, 600
+    ws = [(_dev(oracle.random_blocks(t, n, E, rng), cuda), t) for t, n in zip(types, (4096, 512, 512))]
+    wo = (_dev(oracle.random_blocks(wo_type, E, 4096, rng), cuda), wo_type)
+    g = torch.rand(E, device=cuda) + 0.5
+    x, att, x0 = (torch.randn((T, n), device=cuda) for n in (E, 4096, E))
+    qkv = torch.empty((T, 5120), device=cuda)
+    fa.qkv_proj_rows(*ws, x, g, qkv)
+    y = x0.clone()
+    fa.o_proj_rows(wo, att, y)
+    for n in (16, 17, 32, 33, 63, 480, 481):
+        a = T - n
+        q_part = torch.full((n + 1, 5120), float("nan"), device=cuda)
+        fa.qkv_proj_rows(*ws, x[a:].contiguous(), g, q_part[:n])
+        y_part = torch.cat([x0[a:], x0[:1]])
+        fa.o_proj_rows(wo, att[a:].contiguous(), y_part[:n])
+        torch.cuda.synchronize()
+        assert torch.equal(qkv[a:], q_part[:n]) and torch.isnan(q_part[n]).all(), ("qkv", types, n)
+        assert torch.equal(y[a:], y_part[:n]) and torch.equal(y_part[n], x0[0]), ("o", wo_type, n)
+
+
 def test_projection_rows_gemm_passes_bit_identical(cuda):
     """Beyond 8192 tokens the projections run in passes of 8192 (the workspace's ceiling): each
     token's output does not depend on the batch it came in, so the 8300-token call's rows equal,
