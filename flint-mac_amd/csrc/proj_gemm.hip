@@ -132,30 +132,240 @@ __global__ __launch_bounds__(512) void wprep_kernel(const GemmWeightParams P) {
 // gemm3's three and no weight lo plane, and the scale joins in fp32: acc += s T, one s per weight
 // row and chunk (SUB = 32) or k-step of 16 (SUB = 16); the min as acc -= m S with S = sum_k
 // (xh + xl) over the block, which xprep writes per row and block. The x planes are gemm3's.
-//
-// wprep_int: thread (row n, sub-block b) writes the sub-block's 32 values as f16 into the plane's
-// chunk order (plane_unit), its scales into wd[n / 128][b][32 / SUB][n % 128] and, with mins, its
-// min into wm[n / 128][b][n % 128].
-template <int K, int SUB>
-__global__ __launch_bounds__(256) void wprep_int_kernel(const GemmWeightParams P) {
-    constexpr int NB = K / 32, NS = 32 / SUB;
-    const int idx = blockIdx.x * 256 + threadIdx.x, n = idx / NB, b = idx % NB;  // sub-block fastest
-    const int in2 = P.n_seg > 2 && n >= P.seg[2].row0, in1 = !in2 && P.n_seg > 1 && n >= P.seg[1].row0;
-    const MatvecSeg S = in2 ? P.seg[2] : in1 ? P.seg[1] : P.seg[0];
-    _Float16 v[32];
-    float sc[2], mn;
-    deq32_int(S.type, S.w + (size_t)(n - S.row0) * S.row_bytes, b, v, sc, mn);
+// The rows' bytes are decoded the same way for the planes (wprep_int) and by gemm_raw: a wave stages 32 rows'
+// bytes of a group of blocks in LDS with 16-byte loads along the rows, and a lane decodes the 16 weights
+// of a block that the MFMA takes from it.
+
+// 4 bytes u (0 .. 255) as f16, less `bias` (exact): 0x6400 | u is 1024 + u
+__device__ inline void bytes_f16(uint32_t u, int bias, f16x8 &w, int at) {
+    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+    const h2 off = {(_Float16)(float)(1024 + bias), (_Float16)(float)(1024 + bias)};
+    const h2 a = __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, u, 0x04010400u)) - off;
+    const h2 b = __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, u, 0x04030402u)) - off;
+    w[at] = a[0], w[at + 1] = a[1], w[at + 2] = b[0], w[at + 3] = b[1];
+}
+
+// 8 bytes at p + odd (p 4-byte aligned, odd 0 or 2)
+__device__ inline uint2 lds8(const uint8_t *p, int odd) {
+    const uint32_t *w = (const uint32_t *)p;
+    if (!odd) return make_uint2(w[0], w[1]);
+    return make_uint2(__builtin_amdgcn_alignbit(w[1], w[0], 16), __builtin_amdgcn_alignbit(w[2], w[1], 16));
+}
+
+// The GGUF rows in groups of G chunks: UNITS 16-byte units of a row a group, the last of them at byte
+// LAST of the group's BYTES (whole units but for q6_K, whose last unit overlaps the one before), in LDS
+// rows of STRIDE bytes (an odd number of units, so that the 32 rows' reads of one place spread over the
+// banks). get: lane (row, half h)'s elements 8 h .. 8 h + 7 and 16 + 8 h .. 16 + 8 h + 7 of the group's
+// block j (a constant once unrolled), from its row in LDS: the values (deq32_int's), the scales of
+// elements 0-15 and 16-31, and the min, computed as deq32_int computes them.
+template <int TYPE>
+struct RawRows;
+
+template <>
+struct RawRows<W_Q8_0> {
+    static constexpr int G = 8, BYTES = 272, UNITS = 17, LAST = 256, STRIDE = 272;
+    __device__ static inline void get(const uint8_t *row, int j, int h, f16x8 (&w)[2], float (&sc)[2], float &) {
+        const int odd = j & 1 ? 0 : 2;  // the block's values start at + 2
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-        f16x8 u;
-#pragma unroll
-        for (int e = 0; e < 8; e++) u[e] = v[8 * j + e];
-        *(f16x8 *)(P.wh + plane_unit(n, 4 * b + j, K)) = u;
+        for (int s = 0; s < 2; s++) {
+            const uint2 v = lds8(row + 34 * j + 2 - odd + 16 * s + 8 * h, odd);
+            bytes_f16(v.x ^ 0x80808080u, 128, w[s], 0);
+            bytes_f16(v.y ^ 0x80808080u, 128, w[s], 4);
+        }
+        sc[0] = sc[1] = h2f(*(const uint16_t *)(row + 34 * j));
     }
-    float *const d = P.wd + (((size_t)(n >> 7) * NB + b) * NS) * GEMM_TILE + (n & 127);
-    d[0] = sc[0];  // SUB = 32: the two halves' scales are one
-    if constexpr (NS == 2) d[GEMM_TILE] = sc[1];
-    if (P.imin) P.wm[((size_t)(n >> 7) * NB + b) * GEMM_TILE + (n & 127)] = mn;
+};
+template <>
+struct RawRows<W_Q5_K> {
+    static constexpr int G = 8, BYTES = 176, UNITS = 11, LAST = 160, STRIDE = 176;
+    __device__ static inline void get(const uint8_t *row, int j, int h, f16x8 (&w)[2], float (&sc)[2], float &m) {
+#pragma clang fp contract(off)
+        const u32x4 hdr = *(const u32x4 *)row;
+        const int ls = 4 * (j & 1);
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+            const uint2 qh = *(const uint2 *)(row + 16 + 16 * s + 8 * h);
+            const uint2 ql = *(const uint2 *)(row + 48 + 32 * (j >> 1) + 16 * s + 8 * h);
+            bytes_f16(((ql.x >> ls) & 0x0f0f0f0fu) | (((qh.x >> j) & 0x01010101u) << 4), 0, w[s], 0);
+            bytes_f16(((ql.y >> ls) & 0x0f0f0f0fu) | (((qh.y >> j) & 0x01010101u) << 4), 0, w[s], 4);
+        }
+        // 6-bit scale and min of block j (deq32's)
+        const uint32_t s[3] = {hdr[1], hdr[2], hdr[3]};
+        const uint32_t q = j < 4 ? byte_of(s, j) & 63 : (byte_of(s, j + 4) & 15) | ((byte_of(s, j - 4) >> 6) << 4);
+        const uint32_t mn = j < 4 ? byte_of(s, j + 4) & 63 : (byte_of(s, j + 4) >> 4) | ((byte_of(s, j) >> 6) << 4);
+        sc[0] = sc[1] = h2f(hdr[0] & 0xffff) * (float)q;
+        m = h2f(hdr[0] >> 16) * (float)mn;
+    }
+};
+template <>
+struct RawRows<W_Q6_K> {
+    static constexpr int G = 16, BYTES = 420, UNITS = 27, LAST = 404, STRIDE = 432;
+    __device__ static inline void get(const uint8_t *row, int j, int h, f16x8 (&w)[2], float (&sc)[2], float &) {
+        const int r = j >> 3, n = (j >> 2) & 1, b = j & 3, odd = r ? 2 : 0;  // blocks of 210 bytes
+        const int ls = 4 * (b >> 1), hs = 2 * b;
+        const uint8_t *blk = row + 210 * r - odd;
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+            const uint2 ql = lds8(blk + 64 * n + 32 * (b & 1) + 16 * s + 8 * h, odd);
+            const uint2 qh = lds8(blk + 128 + 32 * n + 16 * s + 8 * h, odd);
+            bytes_f16(((ql.x >> ls) & 0x0f0f0f0fu) | (((qh.x >> hs) & 0x03030303u) << 4), 32, w[s], 0);
+            bytes_f16(((ql.y >> ls) & 0x0f0f0f0fu) | (((qh.y >> hs) & 0x03030303u) << 4), 32, w[s], 4);
+        }
+        // the group's last 4 bytes lie at the end of the overlapping unit
+        const int so = 210 * r + 192 + 2 * (j & 7), end = 16 * UNITS - BYTES;
+        const uint32_t s = *(const uint16_t *)(row + so + (so >= BYTES - 4 ? end : 0));
+        const float d = h2f(*(const uint16_t *)(row + 210 * r + 208 + (r ? end : 0)));
+        sc[0] = d * (float)(int8_t)(s & 0xff), sc[1] = d * (float)(int8_t)(s >> 8);
+    }
+};
+template <>
+struct RawRows<W_IQ4_XS> {
+    static constexpr int G = 16, BYTES = 272, UNITS = 17, LAST = 256, STRIDE = 272;
+    __device__ static inline void get(const uint8_t *row, int j, int h, f16x8 (&w)[2], float (&sc)[2], float &) {
+        const int b = j & 7;
+        const uint2 *blk = (const uint2 *)(row + 136 * (j >> 3)), hdr = blk[0];
+        const uint2 q = blk[1 + 2 * b + h];  // bytes 8 h ..: low nibbles elements 8 h .., high 16 + 8 h ..
+        // the code book + 128 as unsigned bytes
+        constexpr uint32_t X = 0x80808080u, T0 = IQ4_T0 ^ X, T1 = IQ4_T1 ^ X, T2 = IQ4_T2 ^ X, T3 = IQ4_T3 ^ X;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const uint32_t v = (i & 1 ? q.y : q.x) >> (4 * (i >> 1)), sel = v & 0x07070707u;
+            const uint32_t lo = __builtin_amdgcn_perm(T1, T0, sel), hi = __builtin_amdgcn_perm(T3, T2, sel);
+            const uint32_t m = __builtin_amdgcn_perm(0u, 0u, ((v >> 3) & 0x01010101u) | 0x0c0c0c0cu);  // 0xff where bit 3 is set
+            bytes_f16((lo & ~m) | (hi & m), 128, w[i >> 1], 4 * (i & 1));
+        }
+        const uint32_t ls = ((hdr.y >> (8 * (b >> 1) + 4 * (b & 1))) & 15) | (((hdr.x >> (16 + 2 * b)) & 3) << 4);
+        sc[0] = sc[1] = h2f(hdr.x & 0xffff) * (float)((int)ls - 32);
+    }
+};
+template <>
+struct RawRows<W_F16> {
+    static constexpr int G = 4, BYTES = 256, UNITS = 16, LAST = 240, STRIDE = 272;
+    __device__ static inline void get(const uint8_t *row, int j, int h, f16x8 (&w)[2], float (&sc)[2], float &) {
+#pragma unroll
+        for (int s = 0; s < 2; s++) w[s] = *(const f16x8 *)(row + 64 * j + 32 * s + 16 * h);
+        sc[0] = sc[1] = 1.f;
+    }
+};
+template <>
+struct RawRows<W_BF16> {
+    static constexpr int G = 4, BYTES = 256, UNITS = 16, LAST = 240, STRIDE = 272;
+    __device__ static inline void get(const uint8_t *row, int j, int h, f16x8 (&w)[2], float (&sc)[2], float &) {
+        u32x4 q[2];
+        float mx = 0.f;
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+            q[s] = *(const u32x4 *)(row + 64 * j + 32 * s + 16 * h);
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+                mx = fmaxf(mx, fmaxf(fabsf(__uint_as_float(q[s][i] << 16)), fabsf(__uint_as_float(q[s][i] & 0xffff0000u))));
+        }
+        mx = xor32_max(mx);  // the block's largest magnitude: both lane halves
+        const int e = mx > 0.f && __builtin_isfinite(mx) ? __builtin_amdgcn_frexp_expf(mx) - 15 : 0;
+#pragma unroll
+        for (int s = 0; s < 2; s++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                w[s][2 * i] = (_Float16)__builtin_amdgcn_ldexpf(__uint_as_float(q[s][i] << 16), -e);
+                w[s][2 * i + 1] = (_Float16)__builtin_amdgcn_ldexpf(__uint_as_float(q[s][i] & 0xffff0000u), -e);
+            }
+        sc[0] = sc[1] = __builtin_amdgcn_ldexpf(1.f, e);
+    }
+};
+
+constexpr int GR_TILE = 32;  // weight rows of a wave (and tokens of a gemm_raw workgroup)
+
+// A wave's copy of its rows' group bytes into LDS: unit u = 64 i + lane is unit u % UNITS of row u / UNITS
+// of the 32 rows from seg (the first row's byte of the group).
+template <int TYPE>
+struct RawCopy {
+    typedef RawRows<TYPE> RR;
+    static constexpr int NU = GR_TILE * RR::UNITS, WL = (NU + 63) / 64;
+    struct __attribute__((packed, aligned(4))) Unit {
+        u32x4 v;
+    };
+    uint32_t go[WL], lo[WL];
+    u32x4 w[WL];
+    __device__ inline void init(int row_bytes, int lane) {
+#pragma unroll
+        for (int i = 0; i < WL; i++) {
+            const int u = min(64 * i + lane, NU - 1), row = u / RR::UNITS, c = u % RR::UNITS;
+            go[i] = row * row_bytes + (c == RR::UNITS - 1 ? RR::LAST : 16 * c);
+            lo[i] = row * RR::STRIDE + 16 * c;
+        }
+    }
+    __device__ inline void load(const uint8_t *seg) {
+#pragma unroll
+        for (int i = 0; i < WL; i++) w[i] = ((const Unit *)(seg + go[i]))->v;
+    }
+    __device__ inline void store(uint8_t *area, int lane) const {
+#pragma unroll
+        for (int i = 0; i < WL; i++)
+            if (NU % 64 == 0 || i < WL - 1 || 64 * i + lane < NU) *(u32x4 *)(area + lo[i]) = w[i];
+    }
+};
+__device__ inline void wave_lds_fence() {  // the wave's LDS stores before its LDS loads
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// wprep_int: a wave writes 32 rows x 256 elements (512 for the types whose groups are 16 blocks): the values as
+// f16 into the plane's chunk order (plane_unit: lane's k-step s of a block is unit 64 s + lane, so a
+// store writes 1 KiB), the scales into wd[n / 128][b][32 / SUB][n % 128] and, with mins, its min into
+// wm[n / 128][b][n % 128]. HBM-bound: 11.1 MB in and 21.6 MB out for q/k/v in q8_0. (A thread a block, its
+// row bytes read 2 at a time and its 16-byte units written to lines of their own: 12.2 + 12.5 us for a layer's
+// q/k/v and o, q6_K 14.5 + 16.0; now 9.4 + 9.1 and 9.3 + 9.7.)
+constexpr int WP_WAVES = 4;
+template <int SUB, int TYPE>
+__device__ __forceinline__ void wprep_int_wave(const GemmWeightParams &P, const MatvecSeg &S, uint8_t *area, int n0, int item, int K) {
+    typedef RawRows<TYPE> RR;
+    constexpr int G = RR::G, GROUPS = G < 8 ? 8 / G : 1;
+    if (G == 16 && (item & 1)) return;  // the even items take 512 elements
+    const int lane = threadIdx.x & 63, h = lane >> 5, r32 = lane & 31, NB = K / 32;
+    const uint8_t *const row0 = S.w + (size_t)(n0 - S.row0) * S.row_bytes;
+    RawCopy<TYPE> C;
+    C.init(S.row_bytes, lane);
+#pragma unroll
+    for (int q = 0; q < GROUPS; q++) {
+        const int b0 = 8 * item + G * q;  // first block
+        C.load(row0 + (size_t)(b0 / G) * RR::BYTES);
+        if (q > 0) wave_lds_fence();
+        C.store(area, lane);
+        wave_lds_fence();
+#pragma unroll
+        for (int j = 0; j < G; j++) {
+            f16x8 w[2];
+            float sc[2], m = 0.f;
+            RR::get(area + r32 * RR::STRIDE, j, h, w, sc, m);
+            const int b = b0 + j;
+            _Float16 *const o = P.wh + (((size_t)(n0 >> 7) * NB + b) * 512 + ((n0 >> 5) & 3) * 128 + lane) * 8;
+            *(f16x8 *)o = w[0];
+            *(f16x8 *)(o + 512) = w[1];
+            float *const d = P.wd + ((size_t)(n0 >> 7) * NB + b) * (32 / SUB) * GEMM_TILE + (n0 & 127) + r32;
+            if (SUB == 16 || h == 0) d[SUB == 16 ? GEMM_TILE * h : 0] = h == 0 ? sc[0] : sc[1];  // SUB = 32: they are one
+            if (P.imin && h == 0) P.wm[((size_t)(n0 >> 7) * NB + b) * GEMM_TILE + (n0 & 127) + r32] = m;
+        }
+    }
+}
+template <int SUB>
+__global__ __launch_bounds__(64 * WP_WAVES) void wprep_int_kernel(const GemmWeightParams P, int K) {
+    constexpr int AREA = GR_TILE * (SUB == 16 ? RawRows<W_Q6_K>::STRIDE : RawRows<W_Q8_0>::STRIDE);
+    __shared__ __align__(16) uint8_t lds[WP_WAVES][AREA];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n0 = blockIdx.y * GR_TILE, item = blockIdx.x * WP_WAVES + wave;
+    const MatvecSeg s0 = P.seg[0], s1 = P.seg[1], s2 = P.seg[2];
+    const bool in2 = P.n_seg > 2 && n0 >= s2.row0, in1 = !in2 && P.n_seg > 1 && n0 >= s1.row0;
+    const MatvecSeg S = in2 ? s2 : in1 ? s1 : s0;
+    switch (S.type) {
+        case W_Q8_0: wprep_int_wave<SUB, W_Q8_0>(P, S, lds[wave], n0, item, K); break;
+        case W_Q5_K: wprep_int_wave<SUB, W_Q5_K>(P, S, lds[wave], n0, item, K); break;
+        case W_IQ4_XS: wprep_int_wave<SUB, W_IQ4_XS>(P, S, lds[wave], n0, item, K); break;
+        case W_F16: wprep_int_wave<SUB, W_F16>(P, S, lds[wave], n0, item, K); break;
+        case W_BF16: wprep_int_wave<SUB, W_BF16>(P, S, lds[wave], n0, item, K); break;
+        default:
+            if constexpr (SUB == 16) wprep_int_wave<SUB, W_Q6_K>(P, S, lds[wave], n0, item, K);
+    }
 }
 
 __device__ inline double group_ss(const float (&v)[8]) {
@@ -727,145 +937,7 @@ static void launch_gemm_int(const GemmParams &G, hipStream_t stream) {
 // fetched whole lines for a quarter of their bytes and evicted each other's from the L1 (an unsegmented
 // form of this kernel at 512 tokens 121 us against 71 without those loads).
 
-// 4 bytes u (0 .. 255) as f16, less `bias` (exact): 0x6400 | u is 1024 + u
-__device__ inline void bytes_f16(uint32_t u, int bias, f16x8 &w, int at) {
-    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-    const h2 off = {(_Float16)(float)(1024 + bias), (_Float16)(float)(1024 + bias)};
-    const h2 a = __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, u, 0x04010400u)) - off;
-    const h2 b = __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, u, 0x04030402u)) - off;
-    w[at] = a[0], w[at + 1] = a[1], w[at + 2] = b[0], w[at + 3] = b[1];
-}
-
-// 8 bytes at p + odd (p 4-byte aligned, odd 0 or 2)
-__device__ inline uint2 lds8(const uint8_t *p, int odd) {
-    const uint32_t *w = (const uint32_t *)p;
-    if (!odd) return make_uint2(w[0], w[1]);
-    return make_uint2(__builtin_amdgcn_alignbit(w[1], w[0], 16), __builtin_amdgcn_alignbit(w[2], w[1], 16));
-}
-
-// The GGUF rows in groups of G chunks: UNITS 16-byte units of a row a group, the last of them at byte
-// LAST of the group's BYTES (whole units but for q6_K, whose last unit overlaps the one before), in LDS
-// rows of STRIDE bytes (an odd number of units, so that the 32 rows' reads of one place spread over the
-// banks). get: lane (row, half h)'s elements 8 h .. 8 h + 7 and 16 + 8 h .. 16 + 8 h + 7 of the group's
-// block j (a constant once unrolled), from its row in LDS: the values (deq32_int's), the scales of
-// elements 0-15 and 16-31, and the min, computed as deq32_int computes them.
-template <int TYPE>
-struct RawRows;
-
-template <>
-struct RawRows<W_Q8_0> {
-    static constexpr int G = 8, BYTES = 272, UNITS = 17, LAST = 256, STRIDE = 272;
-    __device__ static inline void get(const uint8_t *row, int j, int h, f16x8 (&w)[2], float (&sc)[2], float &) {
-        const int odd = j & 1 ? 0 : 2;  // the block's values start at + 2
-#pragma unroll
-        for (int s = 0; s < 2; s++) {
-            const uint2 v = lds8(row + 34 * j + 2 - odd + 16 * s + 8 * h, odd);
-            bytes_f16(v.x ^ 0x80808080u, 128, w[s], 0);
-            bytes_f16(v.y ^ 0x80808080u, 128, w[s], 4);
-        }
-        sc[0] = sc[1] = h2f(*(const uint16_t *)(row + 34 * j));
-    }
-};
-template <>
-struct RawRows<W_Q5_K> {
-    static constexpr int G = 8, BYTES = 176, UNITS = 11, LAST = 160, STRIDE = 176;
-    __device__ static inline void get(const uint8_t *row, int j, int h, f16x8 (&w)[2], float (&sc)[2], float &m) {
-#pragma clang fp contract(off)
-        const u32x4 hdr = *(const u32x4 *)row;
-        const int ls = 4 * (j & 1);
-#pragma unroll
-        for (int s = 0; s < 2; s++) {
-            const uint2 qh = *(const uint2 *)(row + 16 + 16 * s + 8 * h);
-            const uint2 ql = *(const uint2 *)(row + 48 + 32 * (j >> 1) + 16 * s + 8 * h);
-            bytes_f16(((ql.x >> ls) & 0x0f0f0f0fu) | (((qh.x >> j) & 0x01010101u) << 4), 0, w[s], 0);
-            bytes_f16(((ql.y >> ls) & 0x0f0f0f0fu) | (((qh.y >> j) & 0x01010101u) << 4), 0, w[s], 4);
-        }
-        // 6-bit scale and min of block j (deq32's)
-        const uint32_t s[3] = {hdr[1], hdr[2], hdr[3]};
-        const uint32_t q = j < 4 ? byte_of(s, j) & 63 : (byte_of(s, j + 4) & 15) | ((byte_of(s, j - 4) >> 6) << 4);
-        const uint32_t mn = j < 4 ? byte_of(s, j + 4) & 63 : (byte_of(s, j + 4) >> 4) | ((byte_of(s, j) >> 6) << 4);
-        sc[0] = sc[1] = h2f(hdr[0] & 0xffff) * (float)q;
-        m = h2f(hdr[0] >> 16) * (float)mn;
-    }
-};
-template <>
-struct RawRows<W_Q6_K> {
-    static constexpr int G = 16, BYTES = 420, UNITS = 27, LAST = 404, STRIDE = 432;
-    __device__ static inline void get(const uint8_t *row, int j, int h, f16x8 (&w)[2], float (&sc)[2], float &) {
-        const int r = j >> 3, n = (j >> 2) & 1, b = j & 3, odd = r ? 2 : 0;  // blocks of 210 bytes
-        const int ls = 4 * (b >> 1), hs = 2 * b;
-        const uint8_t *blk = row + 210 * r - odd;
-#pragma unroll
-        for (int s = 0; s < 2; s++) {
-            const uint2 ql = lds8(blk + 64 * n + 32 * (b & 1) + 16 * s + 8 * h, odd);
-            const uint2 qh = lds8(blk + 128 + 32 * n + 16 * s + 8 * h, odd);
-            bytes_f16(((ql.x >> ls) & 0x0f0f0f0fu) | (((qh.x >> hs) & 0x03030303u) << 4), 32, w[s], 0);
-            bytes_f16(((ql.y >> ls) & 0x0f0f0f0fu) | (((qh.y >> hs) & 0x03030303u) << 4), 32, w[s], 4);
-        }
-        // the group's last 4 bytes lie at the end of the overlapping unit
-        const int so = 210 * r + 192 + 2 * (j & 7), end = 16 * UNITS - BYTES;
-        const uint32_t s = *(const uint16_t *)(row + so + (so >= BYTES - 4 ? end : 0));
-        const float d = h2f(*(const uint16_t *)(row + 210 * r + 208 + (r ? end : 0)));
-        sc[0] = d * (float)(int8_t)(s & 0xff), sc[1] = d * (float)(int8_t)(s >> 8);
-    }
-};
-template <>
-struct RawRows<W_IQ4_XS> {
-    static constexpr int G = 16, BYTES = 272, UNITS = 17, LAST = 256, STRIDE = 272;
-    __device__ static inline void get(const uint8_t *row, int j, int h, f16x8 (&w)[2], float (&sc)[2], float &) {
-        const int b = j & 7;
-        const uint2 *blk = (const uint2 *)(row + 136 * (j >> 3)), hdr = blk[0];
-        const uint2 q = blk[1 + 2 * b + h];  // bytes 8 h ..: low nibbles elements 8 h .., high 16 + 8 h ..
-        // the code book + 128 as unsigned bytes
-        constexpr uint32_t X = 0x80808080u, T0 = IQ4_T0 ^ X, T1 = IQ4_T1 ^ X, T2 = IQ4_T2 ^ X, T3 = IQ4_T3 ^ X;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const uint32_t v = (i & 1 ? q.y : q.x) >> (4 * (i >> 1)), sel = v & 0x07070707u;
-            const uint32_t lo = __builtin_amdgcn_perm(T1, T0, sel), hi = __builtin_amdgcn_perm(T3, T2, sel);
-            const uint32_t m = __builtin_amdgcn_perm(0u, 0u, ((v >> 3) & 0x01010101u) | 0x0c0c0c0cu);  // 0xff where bit 3 is set
-            bytes_f16((lo & ~m) | (hi & m), 128, w[i >> 1], 4 * (i & 1));
-        }
-        const uint32_t ls = ((hdr.y >> (8 * (b >> 1) + 4 * (b & 1))) & 15) | (((hdr.x >> (16 + 2 * b)) & 3) << 4);
-        sc[0] = sc[1] = h2f(hdr.x & 0xffff) * (float)((int)ls - 32);
-    }
-};
-template <>
-struct RawRows<W_F16> {
-    static constexpr int G = 4, BYTES = 256, UNITS = 16, LAST = 240, STRIDE = 272;
-    __device__ static inline void get(const uint8_t *row, int j, int h, f16x8 (&w)[2], float (&sc)[2], float &) {
-#pragma unroll
-        for (int s = 0; s < 2; s++) w[s] = *(const f16x8 *)(row + 64 * j + 32 * s + 16 * h);
-        sc[0] = sc[1] = 1.f;
-    }
-};
-template <>
-struct RawRows<W_BF16> {
-    static constexpr int G = 4, BYTES = 256, UNITS = 16, LAST = 240, STRIDE = 272;
-    __device__ static inline void get(const uint8_t *row, int j, int h, f16x8 (&w)[2], float (&sc)[2], float &) {
-        u32x4 q[2];
-        float mx = 0.f;
-#pragma unroll
-        for (int s = 0; s < 2; s++) {
-            q[s] = *(const u32x4 *)(row + 64 * j + 32 * s + 16 * h);
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-                mx = fmaxf(mx, fmaxf(fabsf(__uint_as_float(q[s][i] << 16)), fabsf(__uint_as_float(q[s][i] & 0xffff0000u))));
-        }
-        mx = xor32_max(mx);  // the block's largest magnitude: both lane halves
-        const int e = mx > 0.f && __builtin_isfinite(mx) ? __builtin_amdgcn_frexp_expf(mx) - 15 : 0;
-#pragma unroll
-        for (int s = 0; s < 2; s++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                w[s][2 * i] = (_Float16)__builtin_amdgcn_ldexpf(__uint_as_float(q[s][i] << 16), -e);
-                w[s][2 * i + 1] = (_Float16)__builtin_amdgcn_ldexpf(__uint_as_float(q[s][i] & 0xffff0000u), -e);
-            }
-        sc[0] = sc[1] = __builtin_amdgcn_ldexpf(1.f, e);
-    }
-};
-
 constexpr int XPREP_FEW_ROWS = 512;  // see xprep_row_kernel
-constexpr int GR_TILE = 32;                 // weight rows and tokens per workgroup
 constexpr int GR_CHUNKS = GEMM_SEG / 32;    // chunks of a segment
 static_assert(GR_TILE == GEMM_RAW_TILE, "the x planes hold whole token tiles");
 
@@ -888,29 +960,8 @@ __device__ __forceinline__ void gemm_raw_segment(const GemmParams &P, const uint
     constexpr int NS = 32 / SUB, G = RR::G, NG = GR_CHUNKS / G, XD = 4;
     constexpr bool MIN = TYPE == W_Q5_K;
     const int lane = threadIdx.x & 63, h = lane >> 5, r32 = lane & 31;
-    // row bytes: unit u = 64 i + lane of a group is unit u % UNITS of row u / UNITS
-    constexpr int NU = 32 * RR::UNITS, WL = (NU + 63) / 64;
-    uint32_t go[WL], lo[WL];
-#pragma unroll
-    for (int i = 0; i < WL; i++) {
-        const int u = min(64 * i + lane, NU - 1), row = u / RR::UNITS, c = u % RR::UNITS;
-        go[i] = row * row_bytes + (c == RR::UNITS - 1 ? RR::LAST : 16 * c);
-        lo[i] = row * RR::STRIDE + 16 * c;
-    }
-    struct __attribute__((packed, aligned(4))) Unit {
-        u32x4 v;
-    };
-    u32x4 W[WL];  // the group after the one in LDS
-    auto wload = [&](int q) {
-        const uint8_t *const grp = seg + q * RR::BYTES;
-#pragma unroll
-        for (int i = 0; i < WL; i++) W[i] = ((const Unit *)(grp + go[i]))->v;
-    };
-    auto wstore = [&]() {
-#pragma unroll
-        for (int i = 0; i < WL; i++)
-            if (NU % 64 == 0 || i < WL - 1 || 64 * i + lane < NU) *(u32x4 *)(area + lo[i]) = W[i];
-    };
+    RawCopy<TYPE> C;  // the group after the one in LDS
+    C.init(row_bytes, lane);
     // x: the tile's units of a chunk are 2 KiB of each plane (plane_unit), lane's k-step s at 64 s + lane
     const size_t xo = ((size_t)(t0 >> 7) * (P.K / 32) + chunk0) * (512 * 16) + ((t0 >> 5) & 3) * 2048;
     const uint8_t *const xp[2] = {(const uint8_t *)P.xh + xo, (const uint8_t *)P.xl + xo};
@@ -934,7 +985,7 @@ __device__ __forceinline__ void gemm_raw_segment(const GemmParams &P, const uint
     };
     f32x4 S0, S1;
     uint8_t *const sums = area + 32 * RR::STRIDE;  // [chunk][token]
-    wload(0);
+    C.load(seg);
     if (MIN) {
         const float *const sp = P.xs + ((size_t)(t0 >> 7) * (P.K / 32) + chunk0 + (lane >> 3)) * GEMM_TILE + (t0 & 127) + 4 * (lane & 7);
         S0 = *(const f32x4 *)sp, S1 = *(const f32x4 *)(sp + 8 * GEMM_TILE);
@@ -946,12 +997,10 @@ __device__ __forceinline__ void gemm_raw_segment(const GemmParams &P, const uint
     for (int c = 0; c < GR_CHUNKS; c++) {
         const int q = c / G, j = c % G;
         if (j == 0) {
-            wstore();
+            C.store(area, lane);
             if (MIN && q == 0) *(f32x4 *)(sums + 16 * lane) = S0, *(f32x4 *)(sums + 1024 + 16 * lane) = S1;
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            if (q + 1 < NG) wload(q + 1);
+            wave_lds_fence();
+            if (q + 1 < NG) C.load(seg + (q + 1) * RR::BYTES);
         }
         f16x8 w[2];
         float m = 0.f;
@@ -1060,12 +1109,9 @@ hipError_t launch_proj_gemm(const GemmWeightParams &W, const GemmActParams &X, c
     }
     if (X.T_pad % GM_TILE != 0) return hipErrorInvalidValue;
     if (G.isub == 32 || G.isub == 16) {
-        const bool s32 = G.isub == 32;
-        if (prep_weights) {
-            void (*wk)(GemmWeightParams) = G.K == 2048 ? (s32 ? wprep_int_kernel<2048, 32> : wprep_int_kernel<2048, 16>)
-                                                       : (s32 ? wprep_int_kernel<4096, 32> : wprep_int_kernel<4096, 16>);
-            hipLaunchKernelGGL(wk, dim3(G.N * (G.K / 32) / 256), dim3(256), 0, stream, W);
-        }
+        if (prep_weights)
+            hipLaunchKernelGGL(G.isub == 32 ? wprep_int_kernel<32> : wprep_int_kernel<16>, dim3(G.K / 256 / WP_WAVES, G.N / GR_TILE),
+                               dim3(64 * WP_WAVES), 0, stream, W, G.K);
         if (X.T_pad > 0) {
             if (G.K == 2048)
                 hipLaunchKernelGGL(xprep_kernel<2048>, dim3(X.T_pad / 8), dim3(512), 0, stream, X);
