@@ -490,12 +490,11 @@ __global__ __launch_bounds__(PF_THREADS, 1) void flash_prefill_kernel(const Pref
     // 32-key tiles of this block, then of this split (P.tps tiles each)
     const int tb_lo = (k_lo - P.kbase) >> 5, tb_hi = (q_last - P.kbase) >> 5;
     const int t_lo = tb_lo + split * P.tps, t_hi = min(tb_hi, t_lo + P.tps - 1);
+    if (t_lo > t_hi) return;  // wave-uniform: a split past this block's keys (shorter blocks of a causal layer)
+    // a block whose tiles are one split's writes its output rows itself (prefill_combine_kernel skips them)
+    const bool whole = tb_hi - tb_lo < P.tps;
     // the record of row t, head hq of this split (acc[128], m in log2 units, l)
     auto part_row = [&](int t) { return P.part + ((size_t)(split * P.T + t) * N_HEAD + hq) * PF_PART_STRIDE; };
-    if (t_lo > t_hi) {  // wave-uniform: a split past this block's keys (shorter blocks of a causal layer)
-        if (hh == 0 && row_ok) *(float2 *)(part_row(my_t) + HEAD_DIM) = make_float2(P.sinks[hq] * LOG2E, 0.f);
-        return;
-    }
     const _Float16 *__restrict__ skv = P.sk + (size_t)kvh * (P.k_rows >> 5) * (16 * 64 * 8);
     // Tile t (32 keys from kbase + 32 t): from the attention copy, or for t < n_direct (whole
     // tiles of cached positions of an f16 cache, whose copy would hold the same bits) from the
@@ -629,7 +628,7 @@ __global__ __launch_bounds__(PF_THREADS, 1) void flash_prefill_kernel(const Pref
 
     // m starts at the sink; l counts the sink once (l = 1) unless the keys are split, in which
     // case the merge adds it
-    float m = P.sinks[hq] * LOG2E, l = hh == 0 && n_split == 1 ? 1.f : 0.f;
+    float m = P.sinks[hq] * LOG2E, l = hh == 0 && whole ? 1.f : 0.f;
     f32x16 negm;  // -m in every element: the C operand of each tile's first score MFMA
 #pragma unroll
     for (int e = 0; e < 16; e++) negm[e] = -m;
@@ -811,8 +810,8 @@ __global__ __launch_bounds__(PF_THREADS, 1) void flash_prefill_kernel(const Pref
     //      256 bytes ----
     // split keys: the unnormalised partial (acc in true units, m, l) goes to this split's records
     const float lsum = xor32_sum(l);
-    const float inv = __builtin_amdgcn_ldexpf(n_split == 1 ? 1.0f / lsum : 1.0f, E);  // rows past T: l = 1, acc = 0
-    if (n_split > 1 && hh == 0 && row_ok) *(float2 *)(part_row(my_t) + HEAD_DIM) = make_float2(m, lsum);
+    const float inv = __builtin_amdgcn_ldexpf(whole ? 1.0f / lsum : 1.0f, E);  // rows past T: l = 1, acc = 0
+    if (!whole && hh == 0 && row_ok) *(float2 *)(part_row(my_t) + HEAD_DIM) = make_float2(m, lsum);
     float4 *const ob = (float4 *)&q_lds[wave][0][0];
 #pragma unroll
     for (int half = 0; half < 2; half++) {
@@ -829,7 +828,7 @@ __global__ __launch_bounds__(PF_THREADS, 1) void flash_prefill_kernel(const Pref
             const int r = 4 * i + (lane >> 4), c = lane & 15;
             const float4 v = ob[r * 16 + (c ^ (r & 15))];
             if (t0 + r < P.T) {
-                float *dst = n_split == 1 ? P.att + (size_t)(t0 + r) * Q_DIM + hq * HEAD_DIM : part_row(t0 + r);
+                float *dst = whole ? P.att + (size_t)(t0 + r) * Q_DIM + hq * HEAD_DIM : part_row(t0 + r);
                 // streaming stores: the output is not read again here, and left in the caches it
                 // would evict the K/V tiles the other workgroups of the XCD still read (measured
                 // 1.5-2.5 us faster per call on both layer kinds; q read the same way was slower)
@@ -841,12 +840,18 @@ __global__ __launch_bounds__(PF_THREADS, 1) void flash_prefill_kernel(const Pref
 
 // Merge of a split prefill (fused.metal:331-350 per query row): one wave per (row t, head),
 // lane l holds dims 2l, 2l + 1 and the (m, l) pair of split l; the records are read 8 splits
-// at a time (indices past n_split repeat the last one with weight 0); splits with l = 0 (no
-// key of the row) get weight 0 and are skipped.
+// at a time (indices past the block's last split repeat it with weight 0); splits with l = 0 (no
+// key of the row) get weight 0 and are skipped. Rows of blocks of one split are the flash kernel's.
 __global__ __launch_bounds__(256) void prefill_combine_kernel(const PrefillParams P) {
     const int lane = threadIdx.x & 63, pair = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (pair >= P.T * N_HEAD) return;
-    const int t = pair / N_HEAD, hq = pair % N_HEAD, ns = P.n_split;
+    const int t = pair / N_HEAD, hq = pair % N_HEAD;
+    // the row's query block, its tiles and its splits, as flash_prefill_kernel has them
+    const int t0 = t / PF_BQ * PF_BQ, q_first = P.p0 + t0, q_last = P.p0 + min(t0 + PF_BQ, P.T) - 1;
+    const int k_lo = P.is_swa ? max(P.kbase, q_first - (P.window - 1)) : 0;
+    const int tiles = ((q_last - P.kbase) >> 5) - ((k_lo - P.kbase) >> 5) + 1;
+    const int ns = __builtin_popcountll(__builtin_amdgcn_ballot_w64(lane * P.tps < tiles));  // at most PF_MAX_SPLIT, 64
+    if (ns <= 1) return;  // wave-uniform
     const float *rec = P.part + ((size_t)t * N_HEAD + hq) * PF_PART_STRIDE;
     const size_t sstride = (size_t)P.T * N_HEAD * PF_PART_STRIDE;
     const float sink = P.sinks[hq] * LOG2E;

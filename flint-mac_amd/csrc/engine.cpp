@@ -289,20 +289,33 @@ void prefill_impl(const flint_attn_layer *L, const float *qkv, int q_stride, int
     uint32_t id = ++next_call;
     if (id == 0) id = ++next_call;
     P.call_id = id;
-    // Key splits when the grid of (query block, kv head) workgroups would leave most CUs idle on
-    // a long key range (a short prefill at a long context: one workgroup per kv head would stream
-    // the whole cache through one CU). Splits of the longest block's tiles, 8 at least, so the
-    // launch has about 512 workgroups; the merge kernel adds the sink.
+    // Key splits when the grid of (query block, kv head) workgroups would leave CUs idle on a long key
+    // range (a short prefill at a long context: one workgroup per kv head would stream the whole
+    // cache through one CU); the merge kernel adds the sink. A split costs a q prologue (~8 us, 9
+    // tiles' time) and its records, so:
+    //  * the splits' workgroups fit one round of the 256 CUs (200 tokens at 4000 cached 39 us, with two rounds
+    //    52; 64 at 16000 40 and 56), and no split is made where the grid nearly fills the round by itself
+    //    (2000 tokens at 2000: 150 and 187 us);
+    //  * unless every split of two rounds still has 31 tiles: the rounds' ends then
+    //    overlap (700 tokens at 10000: 193 us with one round, 149 with two; 1339 at 4557: 190 and 164);
+    //  * from 256 tokens on, ranges of under 32 tiles stay whole: the records cost more than the tiles saved
+    //    (SWA: 1000 tokens 54 us in two splits, 29 whole; 2000 96 and 34);
+    //  * the shorter the batch, the fewer tiles a split may have (records are per token).
     {
         const int nqb = (T + 31) / 32;
         // tiles of the longest query block: the last one on a full layer; on an SWA layer at
         // most the 18 tiles that a 32-query block's window [first - (window - 1), first + 31] spans
         const int longest = L->is_swa ? std::min(((p0 + T - 1 - P.kbase) >> 5) + 1, (L->window + 62) / 32 + 1)
                                       : ((p0 + T - 1) >> 5) + 1;
+        constexpr int CUS = 256;
         const int base = nqb * N_HEAD_KV;
-        int ns = 1;
-        if (base < 256 && longest >= 16)
-            ns = std::min({PF_MAX_SPLIT, (512 + base - 1) / base, (longest + 7) / 8});
+        int ns = base >= CUS * 7 / 8 ? 1 : CUS / base;
+        // two rounds, or the splits of a started third where two would leave over a sixth of their slots idle
+        const int n2 = 2 * CUS / base * base * 6 >= 2 * CUS * 5 ? 2 * CUS / base : (2 * CUS + base - 1) / base;
+        if (base < CUS * 7 / 8 && longest >= 31 * n2) ns = n2;
+        const int min_tiles = T > 64 ? 8 : T > 16 ? (longest < 32 ? 4 : longest < 64 ? 6 : 8) : longest < 32 ? 2 : 4;
+        ns = std::min({PF_MAX_SPLIT, ns, (longest + min_tiles - 1) / min_tiles});
+        if (T > 256 && longest < 32) ns = 1;
         const int tps = (longest + ns - 1) / ns;
         P.n_split = (longest + tps - 1) / tps;
         P.tps = P.n_split > 1 ? tps : 1 << 24;

@@ -156,8 +156,10 @@ __device__ inline uint2 lds8(const uint8_t *p, int odd) {
 // LAST of the group's BYTES (whole units but for q6_K, whose last unit overlaps the one before), in LDS
 // rows of STRIDE bytes (an odd number of units, so that the 32 rows' reads of one place spread over the
 // banks). get: lane (row, half h)'s elements 8 h .. 8 h + 7 and 16 + 8 h .. 16 + 8 h + 7 of the group's
-// block j (a constant once unrolled), from its row in LDS: the values (deq32_int's), the scales of
-// elements 0-15 and 16-31, and the min, computed as deq32_int computes them.
+// block j (a constant once unrolled), from its row in LDS: the values, the scales of elements
+// 0-15 and 16-31, and the min, in ggml's float order, so that scale * value - min is deq32's weight
+// (f16: scale 1; bf16: 8 significant bits, exact in f16 once the block's largest magnitude is scaled into
+// [2^14, 2^15): values below 2^-10 of it, beneath f16's normal range, round to f16's subnormal steps).
 template <int TYPE>
 struct RawRows;
 

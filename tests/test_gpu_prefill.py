@@ -359,6 +359,31 @@ def test_prefill_short_at_long_context_split_keys(cuda, store, is_swa):
         p += T
 
 
+@pytest.mark.parametrize("store", ["f16", "bf16"])
+@pytest.mark.parametrize("T,p0", [(1000, 0), (520, 33), (33, 63), (90, 991)])
+def test_prefill_blocks_whole_and_split(cuda, store, T, p0):
+    """Causal calls whose shorter query blocks fit one key split and write their rows themselves while the
+    longer ones are split and merged (1000 tokens: 16 whole blocks, 16 of two splits; ragged last
+    blocks), and calls whose blocks all have the same number of splits: every row against the oracle."""
+    rng = np.random.default_rng(T + p0)
+    qn, kn, sk = layer_weights(rng)
+    n = p0 + T
+    kv = fa.KVLayer(is_swa=False, has_rope=True, n_slots=(n + 31) // 32 * 32, kv_dtype=store, rope_theta=1e4, q_norm=qn,
+                    k_norm=kn, sinks=sk)
+    L = oracle_layer(kv, qn, kn, sk, store)
+    qkv = rng.standard_normal((n, QKV_DIM)).astype(np.float32)
+    dq = torch.from_numpy(qkv).to(cuda)
+    att = torch.full((n, Q_DIM), float("nan"), device=cuda)
+    if p0:
+        kv.prefill(dq[:p0], att[:p0], 0)
+    kv.prefill(dq[p0:], att[p0:], p0)
+    torch.cuda.synchronize()
+    K = np.zeros((n, KV_DIM), np.float32)
+    V = np.zeros((n, KV_DIM), np.float32)
+    want = fo.prefill(L, qkv, 0, K, V, n_threads=16)
+    assert_close(att.cpu().numpy(), want, f"T={T} p0={p0} {store}")
+
+
 @pytest.mark.parametrize("is_swa", [False, True], ids=["full", "swa"])
 def test_prefill_f16_cached_tiles_on_scaled_path(cuda, is_swa):
     """An f16 continuation reads its whole cached tiles from the cache itself; with q gains
