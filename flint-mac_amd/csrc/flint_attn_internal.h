@@ -114,7 +114,7 @@ struct MatvecParams {
     float eps;
     float *y;              // [n_tok] rows of y_stride floats: y = W x, or y += W x when add
     int add;
-    int n_tok;             // tokens (grid x), >= 1
+    int n_tok;             // tokens, >= 1
     long long x_stride, y_stride;
 };
 // Rows rows[0 .. n) of a weight tensor (row_bytes each) dequantised into out + i * out_stride.

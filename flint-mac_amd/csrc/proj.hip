@@ -4,7 +4,8 @@
 //     the prefill's embedding, k_embed_rows, prefill.metal:272, engine.mm:1067-1069);
 //   * matvec_kernel: y = W x with 2048- or 4096-element rows, optionally on RMSNorm(x) * g
 //     (the q/k/v projections, engine.mm:728-732) or added to y (o_proj with the residual,
-//     engine.mm:811).
+//     engine.mm:811);
+//   * matvec_tokens_kernel: the same for a few tokens.
 //
 // Formats: ggml's block layouts (/root/reference/third_party/ggml/ggml-common.h), type ids
 // from /root/reference/src/gguf.h:14-19. Every row is cut into 32-element sub-blocks, the
@@ -23,6 +24,8 @@
 // fp32; a wave-wide sum gives y[row].
 // f32/f16/bf16 rows are read straight from HBM (64- or 128-byte sub-blocks, aligned).
 #include <hip/hip_runtime.h>
+
+#include <type_traits>
 
 #include "common.h"
 #include "dequant.h"
@@ -62,7 +65,7 @@ __global__ __launch_bounds__(64) void get_rows_kernel(const RowsParams P) {
 }
 
 // ---------------------------------------------------------------------------
-// matvec: a workgroup of MV_WAVES waves serves MV_WAVES * R consecutive rows of one token.
+// matvec: one token. A workgroup of MV_WAVES waves serves MV_WAVES * R consecutive rows.
 // x (times the RMSNorm gains, when norm_w is given; the norm's scale multiplies the row sums)
 // is read from HBM once per workgroup into LDS; each wave then takes R rows, whose bytes it
 // requested at kernel start, and reads its lanes' 32-element slices of x from LDS.
@@ -115,29 +118,24 @@ __global__ __launch_bounds__(64 * MV_WAVES) void matvec_kernel(const MatvecParam
     // wave index made scalar: the row segment, its type and its row pointer are then known
     // to be wave-uniform (scalar branches for the format, scalar load bases)
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int row0 = (blockIdx.y * MV_WAVES + wave) * R;  // R rows, all in one segment
+    const int row0 = (blockIdx.x * MV_WAVES + wave) * R;  // R rows, all in one segment
     // the segment by selection among constant-index reads: the kernel arguments arrive in one
     // batch of scalar loads (a search loop over P.seg costs a memory round trip per step)
     const MatvecSeg s0 = P.seg[0], s1 = P.seg[1], s2 = P.seg[2];
     const int n_seg = P.n_seg, add = P.add;
-    const long long x_stride = P.x_stride, y_stride = P.y_stride;
-    const float *const x = P.x, *const norm_w = P.norm_w;
-    float *const y = P.y;
+    const float *const xt = P.x, *const norm_w = P.norm_w;
+    float *const yt = P.y;
     const float eps = P.eps;
     pin_sgpr(s0.w), pin_sgpr(s0.type), pin_sgpr(s0.row0), pin_sgpr(s0.row_bytes);
     pin_sgpr(s1.w), pin_sgpr(s1.type), pin_sgpr(s1.row0), pin_sgpr(s1.row_bytes);
     pin_sgpr(s2.w), pin_sgpr(s2.type), pin_sgpr(s2.row0), pin_sgpr(s2.row_bytes);
-    pin_sgpr(n_seg), pin_sgpr(add), pin_sgpr(x_stride), pin_sgpr(y_stride), pin_sgpr(x), pin_sgpr(norm_w);
-    pin_sgpr(y), pin_sgpr(eps);
+    pin_sgpr(n_seg), pin_sgpr(add), pin_sgpr(xt), pin_sgpr(norm_w);
+    pin_sgpr(yt), pin_sgpr(eps);
     __builtin_amdgcn_sched_barrier(0);
     const bool in2 = n_seg > 2 && row0 >= s2.row0, in1 = !in2 && n_seg > 1 && row0 >= s1.row0;
     const MatvecSeg S = in2 ? s2 : in1 ? s1 : s0;
     const uint8_t *wrow = S.w + (size_t)(row0 - S.row0) * S.row_bytes;
     const bool fl = w_is_float(S.type);
-    // token blockIdx.x: consecutive workgroups take the same rows for successive tokens,
-    // so a batch reads each weight row from HBM about once (the rest hit L2)
-    const float *__restrict__ xt = x + (size_t)blockIdx.x * x_stride;
-    float *__restrict__ yt = y + (size_t)blockIdx.x * y_stride;
 
     // x and the gains: XPT consecutive elements per thread, 16-byte loads
     f32x4 xv[XPT / 4], gv[XPT / 4];
@@ -286,26 +284,224 @@ __global__ __launch_bounds__(64 * MV_WAVES) void matvec_kernel(const MatvecParam
     }
 }
 
+// ---------------------------------------------------------------------------
+// matvec_tokens: 2 .. 15 tokens (and longer batches whose output rows the GEMM cannot store) through the
+// same rows. Bound by instruction issue and LDS reads: a token's 64 products a lane need its 8 KB of x.
+// With a workgroup a token, as in matvec_kernel, every token decoded the rows again. Here a wave decodes
+// its rows once into registers (64 weights a lane: two rows of 2048 elements or one of 4096), the workgroup
+// puts the x rows of up to TOKENS tokens into LDS (times the gains) and a wave takes the tokens one after
+// another. Token t's sum goes to lane t: a pass ends with one store a row (and one load, when
+// adding). Every sum has matvec_kernel's terms in its order, so a token has the single-token call's
+// bits. 256 workgroups of 10 (q/k/v) or 8 (o) waves: one round of the CUs; half the waves with twice the
+// rows each, which halves the LDS reads, measured slower (9 tokens 31 us, 15 tokens 39): too few waves to
+// cover the reads' latency. q/k/v + o, a workgroup a token -> here, of which 15.6 us is what two calls cost
+// the host: 9 tokens of q5_K 59.2 -> 24.3 us, of q8_0 35.1 -> 21.2, of bf16 62.3 -> 23.2; 15 tokens of q8_0
+// 52.7 -> 29.4; 2 tokens of q8_0 16.7 -> 15.9, of q5_K 18.4 -> 15.7; 2000 tokens into unaligned rows (q5_K o
+// alone) 4817 -> 1281.
+template <int K>
+struct MtShape;
+template <>
+struct MtShape<2048> {
+    static constexpr int WAVES = 10, R = 2, TOKENS = 15;
+};
+template <>
+struct MtShape<4096> {
+    static constexpr int WAVES = 8, R = 1, TOKENS = 7;
+};
+
+template <int K>
+__global__ __launch_bounds__(64 * MtShape<K>::WAVES) void matvec_tokens_kernel(const MatvecParams P) {
+    constexpr int WAVES = MtShape<K>::WAVES, R = MtShape<K>::R, TOKENS = MtShape<K>::TOKENS;
+    constexpr int SUBS = K / 32 / 64;                  // sub-blocks per lane and row
+    constexpr int QBYTES = K / 32 * 34;                // largest quantised row (q8_0)
+    constexpr int UNITS = (QBYTES / 16 + 63) / 64;     // 16-byte loads per lane for it
+    constexpr int QROW = (QBYTES + 4 + 15) / 16 * 16;  // a staged row, + 4 bytes read past a q8_0 row's end
+    constexpr int XPT = K / 256;                       // x elements per thread: 256 threads a token, as matvec_kernel's
+    static_assert(SUBS * R == 2 && WAVES * R * QROW <= TOKENS * K * 4 && WAVES * 64 >= 512, "shape");
+    __shared__ __align__(16) uint8_t lds[TOKENS * K * 4];  // the rows' bytes, then the x rows
+    __shared__ double part[TOKENS][4];
+    float *const xs = (float *)lds;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int row0 = (blockIdx.x * WAVES + wave) * R;  // R rows, all in one segment
+    const bool rows_ok = row0 < P.n_rows;              // the last workgroup's waves past the rows only stage x
+    const MatvecSeg s0 = P.seg[0], s1 = P.seg[1], s2 = P.seg[2];
+    const bool in2 = P.n_seg > 2 && row0 >= s2.row0, in1 = !in2 && P.n_seg > 1 && row0 >= s1.row0;
+    const MatvecSeg S = in2 ? s2 : in1 ? s1 : s0;
+    const uint8_t *wrow = S.w + (size_t)((rows_ok ? row0 : S.row0) - S.row0) * S.row_bytes;
+    const bool q8 = S.type == W_Q8_0;
+    // this lane's weights: sub-block lane + 64 i of row r at w[r * SUBS + i] (q8_0: the quants, d their scale)
+    float w[2][32], d[2] = {1.f, 1.f};
+    if (w_is_float(S.type)) {
+#pragma unroll
+        for (int k = 0; k < 2; k++) deq32(S.type, wrow + (size_t)(k / SUBS) * S.row_bytes, lane + 64 * (k % SUBS), w[k]);
+    } else {
+        uint8_t *const stage = lds + wave * (R * QROW);
+        const int n_units = S.row_bytes >> 4;
+        u32x4 u[R][UNITS];
+#pragma unroll
+        for (int r = 0; r < R; r++)
+#pragma unroll
+            for (int k = 0; k < UNITS; k++)
+                u[r][k] = ((const u32x4 *)(wrow + (size_t)r * S.row_bytes))[min(lane + 64 * k, n_units - 1)];
+#pragma unroll
+        for (int r = 0; r < R; r++)
+#pragma unroll
+            for (int k = 0; k < UNITS; k++)
+                if (lane + 64 * k < n_units) ((u32x4 *)(stage + r * QROW))[lane + 64 * k] = u[r][k];
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        if (q8) {
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                const int base = 34 * (lane + 64 * (k % SUBS));
+                const bool odd = base & 2;  // the block starts 2 bytes into a word
+                const uint32_t *dw = (const uint32_t *)(stage + (k / SUBS) * QROW + (base & ~3));
+                uint32_t v[9];
+#pragma unroll
+                for (int j = 0; j < 9; j++) v[j] = dw[j];
+                d[k] = h2f(odd ? v[0] >> 16 : v[0] & 0xffffu);
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    const uint32_t q = odd ? v[j + 1] : __builtin_amdgcn_alignbit(v[j + 1], v[j], 16);
+                    w[k][4 * j] = (float)(int8_t)(q & 0xffu);
+                    w[k][4 * j + 1] = (float)(int8_t)((q >> 8) & 0xffu);
+                    w[k][4 * j + 2] = (float)(int8_t)((q >> 16) & 0xffu);
+                    w[k][4 * j + 3] = (float)(int8_t)(q >> 24);
+                }
+            }
+        } else {
+#pragma unroll
+            for (int k = 0; k < 2; k++) deq32(S.type, stage + (k / SUBS) * QROW, lane + 64 * (k % SUBS), w[k]);
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 2; k++)
+#pragma unroll
+        for (int e = 0; e < 32; e++) asm volatile("" : "+v"(w[k][e]));  // decoded here, not once a token
+
+    for (int t0 = 0; t0 < P.n_tok; t0 += TOKENS) {
+        const int n = min(TOKENS, P.n_tok - t0);
+        __syncthreads();  // the rows' bytes, or the pass before's x, have been read
+        // x of tokens t0 .. t0 + n - 1: two at a time, 256 threads each
+        if (tid < 512) {
+            const int u = tid & 255;
+            for (int t = tid >> 8; t < n; t += 2) {
+                const float *xt = P.x + (size_t)(t0 + t) * P.x_stride + XPT * u;
+                f32x4 xv[XPT / 4];
+#pragma unroll
+                for (int k = 0; k < XPT / 4; k++) xv[k] = *(const f32x4 *)(xt + 4 * k);
+                if (P.norm_w) {
+                    double ss = 0;
+#pragma unroll
+                    for (int k = 0; k < XPT / 4; k++)
+#pragma unroll
+                        for (int e = 0; e < 4; e++) ss += (double)xv[k][e] * xv[k][e];
+                    ss = wave_sum_f64(ss);
+                    if (lane == 0) part[t][(tid >> 6) & 3] = ss;
+#pragma unroll
+                    for (int k = 0; k < XPT / 4; k++) {
+                        const f32x4 gv = *(const f32x4 *)(P.norm_w + XPT * u + 4 * k);
+#pragma unroll
+                        for (int e = 0; e < 4; e++) xv[k][e] = xv[k][e] * gv[e];
+                    }
+                }
+#pragma unroll
+                for (int k = 0; k < XPT / 4; k++) *(f32x4 *)&xs[t * K + xs_index(XPT * u + 4 * k)] = xv[k];
+            }
+        }
+        // lane t: token t0 + t's row of y
+        const bool mine = lane < n && rows_ok;
+        float *const y = P.y + (size_t)(t0 + (mine ? lane : 0)) * P.y_stride + row0;
+        float yin[R], out[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) yin[r] = P.add && mine ? y[r] : 0.f, out[r] = 0.f;
+        __syncthreads();
+        float scale = 1.f;
+        if (P.norm_w && lane < n) {
+            double ss = 0;
+#pragma unroll
+            for (int i = 0; i < 4; i++) ss += part[lane][i];
+            scale = 1.0f / sqrtf((float)(ss / K) + P.eps);
+        }
+        auto dots = [&](auto is_q8) {
+            for (int t = 0; t < n; t++) {
+                float acc[R];
+#pragma unroll
+                for (int r = 0; r < R; r++) acc[r] = 0.f;
+#pragma unroll
+                for (int i = 0; i < SUBS; i++) {
+                    float xl[32];
+#pragma unroll
+                    for (int k = 0; k < 8; k++) {
+                        const f32x4 v = *(const f32x4 *)&xs[t * K + xs_index(32 * (lane + 64 * i) + 4 * k)];
+                        xl[4 * k] = v[0], xl[4 * k + 1] = v[1], xl[4 * k + 2] = v[2], xl[4 * k + 3] = v[3];
+                    }
+#pragma unroll
+                    for (int r = 0; r < R; r++) {
+                        const int k = r * SUBS + i;
+                        if constexpr (decltype(is_q8)::value) {
+                            float b0 = 0.f, b1 = 0.f;
+#pragma unroll
+                            for (int j = 0; j < 32; j += 2) b0 = fmaf(w[k][j], xl[j], b0), b1 = fmaf(w[k][j + 1], xl[j + 1], b1);
+                            acc[r] = fmaf(d[k], b0 + b1, acc[r]);
+                        } else {
+#pragma unroll
+                            for (int e = 0; e < 32; e++) acc[r] = fmaf(w[k][e], xl[e], acc[r]);
+                        }
+                    }
+                }
+#pragma unroll
+                for (int r = 0; r < R; r++) {
+                    const float a = wave_sum(acc[r]);
+                    out[r] = lane == t ? a : out[r];
+                }
+            }
+        };
+        if (q8)
+            dots(std::true_type{});
+        else
+            dots(std::false_type{});
+        if (mine)
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                const float a = out[r] * scale;
+                y[r] = P.add ? yin[r] + a : a;
+            }
+    }
+}
+
 hipError_t launch_get_rows(const RowsParams &P, hipStream_t stream) {
     hipLaunchKernelGGL(get_rows_kernel, dim3((P.n_sub + 63) / 64, P.n), dim3(64), 0, stream, P);
     return hipGetLastError();
 }
 
-// Rows per wave: 2 for the 2048-element rows (q/k/v: 640 workgroups per token) and 1 for the
+// Rows per wave: 2 for the 2048-element rows (q/k/v: 640 workgroups) and 1 for the
 // 4096-element rows (o: 512 workgroups, two waves per SIMD: with one, each row's LDS reads and
 // FMA chain were exposed); measured best of 1, 2, 4 and 8 for either.
 constexpr int MV_ROWS_2048 = 2, MV_ROWS_4096 = 1;
+constexpr int MT_MIN_TOKENS = 2;  // at 2 tokens matvec_tokens_kernel is ahead in every type (q5_K 18.4 -> 15.7 us)
 
 int matvec_row_multiple(int k) { return MV_WAVES * (k == 2048 ? MV_ROWS_2048 : MV_ROWS_4096); }
 
 hipError_t launch_matvec(const MatvecParams &P, int k, hipStream_t stream) {
+    if (P.n_tok >= MT_MIN_TOKENS) {
+        if (k == 2048) {
+            constexpr int ROWS = MtShape<2048>::WAVES * MtShape<2048>::R;
+            hipLaunchKernelGGL(matvec_tokens_kernel<2048>, dim3((P.n_rows + ROWS - 1) / ROWS), dim3(64 * MtShape<2048>::WAVES), 0, stream, P);
+        } else {
+            constexpr int ROWS = MtShape<4096>::WAVES * MtShape<4096>::R;
+            hipLaunchKernelGGL(matvec_tokens_kernel<4096>, dim3((P.n_rows + ROWS - 1) / ROWS), dim3(64 * MtShape<4096>::WAVES), 0, stream, P);
+        }
+        return hipGetLastError();
+    }
     const dim3 block(64 * MV_WAVES);
     if (k == 2048)
-        hipLaunchKernelGGL((matvec_kernel<2048, MV_ROWS_2048>), dim3(P.n_tok, P.n_rows / matvec_row_multiple(k)),
-                           block, 0, stream, P);
+        hipLaunchKernelGGL((matvec_kernel<2048, MV_ROWS_2048>), dim3(P.n_rows / matvec_row_multiple(k)), block, 0,
+                           stream, P);
     else
-        hipLaunchKernelGGL((matvec_kernel<4096, MV_ROWS_4096>), dim3(P.n_tok, P.n_rows / matvec_row_multiple(k)),
-                           block, 0, stream, P);
+        hipLaunchKernelGGL((matvec_kernel<4096, MV_ROWS_4096>), dim3(P.n_rows / matvec_row_multiple(k)), block, 0,
+                           stream, P);
     return hipGetLastError();
 }
 

@@ -194,6 +194,37 @@ def test_projection_rows_small_batch_equal_single_token_calls(cuda):
     assert torch.equal(y_rows, y_one)
 
 
+@pytest.mark.parametrize("types,wo_type", [(("q8_0",) * 3, "q8_0"), (("q5_K", "q6_K", "iq4_xs"), "q5_K"),
+                                           (("iq4_xs", "f16", "q6_K"), "iq4_xs"), (("f16", "f32", "q8_0"), "f32"),
+                                           (("bf16",) * 3, "bf16"), (("q6_K",) * 3, "f16")])
+def test_projection_rows_few_tokens_equal_single_token_calls(cuda, types, wo_type):
+    """Batches that share a decoded row among their tokens, at the edges of the kernel's passes (7 and 15
+    tokens) and, with output rows that are not 16-byte aligned, beyond the GEMM's size: every token has the
+    single-token call's bits."""
+    import torch
+    rng = np.random.default_rng(43)
+    T, E = 31, fa.N_EMBD
+    ws = [(_dev(oracle.random_blocks(t, n, E, rng), cuda), t) for t, n in zip(types, (4096, 512, 512))]
+    wo = (_dev(oracle.random_blocks(wo_type, E, 4096, rng), cuda), wo_type)
+    g = torch.rand(E, device=cuda) + 0.5
+    x, att, x0 = (torch.randn((T, n), device=cuda) for n in (E, 4096, E))
+    qkv, y = torch.empty((T, 5120), device=cuda), x0.clone()
+    for t in range(T):
+        fa.qkv_proj(*ws, x[t], g, qkv[t])
+        fa.o_proj(wo, att[t], y[t])
+    for n, odd in ((2, 0), (7, 0), (8, 1), (14, 0), (15, 0), (16, 1), (31, 1)):
+        rows = torch.full((n + 1, 5120 + odd), float("nan"), device=cuda)
+        fa.qkv_proj_rows(*ws, x[:n], g, rows[:n])
+        buf = torch.full((odd + (n + 1) * E,), 3.0, device=cuda)
+        out = buf[odd:].view(n + 1, E)
+        out[:n] = x0[:n]
+        fa.o_proj_rows(wo, att[:n], out[:n])
+        torch.cuda.synchronize()
+        assert torch.equal(rows[:n, :5120], qkv[:n]) and torch.isnan(rows[n]).all(), ("qkv", types, n)
+        assert torch.isnan(rows[:, 5120:]).all()
+        assert torch.equal(out[:n], y[:n]) and (out[n] == 3).all() and (buf[:odd] == 3).all(), ("o", wo_type, n)
+
+
 def _gemm_case(cuda, rng, types, wo_type, T, x_scale=None, att_scale=None):
     """qkv_proj_rows and o_proj_rows on T tokens (the GEMM path) against the oracle's matvec of
     every token, within _rows_bound. x_scale / att_scale: per-row factors for the inputs."""
