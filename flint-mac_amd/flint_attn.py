@@ -146,9 +146,12 @@ def header_functions():
     return sorted(set(names))
 
 
+_ErrText = ctypes.c_char * 512
+
+
 def _call(fn, *args):
-    err = ctypes.create_string_buffer(512)
-    rc = fn(*args, err, len(err))
+    err = _ErrText()
+    rc = fn(*args, err, 512)
     if rc != 0:
         raise FlintAttnError(err.value.decode())
 
@@ -167,7 +170,9 @@ def k_tile_offsets():
 def _stream(stream):
     if stream is None:
         import torch
-        return torch.cuda.current_stream().cuda_stream
+        # the handle of torch.cuda.current_stream() without its Stream object, which took 2.6 of the 7.6 us of a
+        # decode call (0.3 us this way); the device goes through current_device(), which initialises CUDA
+        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
     return stream
 
 

@@ -369,3 +369,20 @@ def test_decode_batch_config5_workload(cuda, store, is_swa):
             ring[np.arange(first, p + 1) & (n_slots - 1)] = ring_hist
             got_ring = kv.v_slots()[s].float().cpu().numpy().transpose(1, 0, 2).reshape(n_slots, KV_DIM)
             assert np.array_equal(got_ring, ring), f"seq {s}: V ring"
+
+
+@pytest.mark.parametrize("side", [False, True])
+def test_calls_go_to_the_current_stream(cuda, side):
+    """Without a stream argument a call goes to torch's current stream, of the calling thread; a given
+    handle is used as it is."""
+    import threading
+    s = torch.cuda.Stream() if side else torch.cuda.default_stream()
+    with torch.cuda.stream(s):
+        assert fa._stream(None) == torch.cuda.current_stream().cuda_stream == s.cuda_stream
+        other = []
+        t = threading.Thread(target=lambda: other.append((fa._stream(None), torch.cuda.current_stream().cuda_stream)))
+        t.start()
+        t.join()
+        assert other[0][0] == other[0][1]
+    assert fa._stream(None) == torch.cuda.current_stream().cuda_stream
+    assert fa._stream(s.cuda_stream) == s.cuda_stream and fa._stream(12) == 12
