@@ -4,15 +4,15 @@
 // (/root/reference/src/metal/prefill.metal:99-266, dispatched per 512-token
 // chunk at /root/reference/src/engine.mm:1087-1104).
 //
-// Three launches per layer call, stream-ordered:
+// Two launches per layer call (and the merge of split keys), stream-ordered:
 //  prefix:  positions [kbase, p0) already in the layer's cache are converted
 //           into the attention copy (f16, below). kbase = 0 for full layers,
 //           max(0, p0 - 512) for SWA layers (the window of the first new token).
 //  kv_prep: per new token, RMSNorm (+ NEOX RoPE) of the 4 k heads and the v
 //           rows, rounded to the cache dtype, into the cache (SWA: only the last
 //           n_slots positions, slot p & (n_slots-1)) and into the attention copy.
-//           The prefix runs first because a long SWA prefill overwrites ring
-//           slots the prefix reads.
+//           The prefix is part of this launch, unless a long SWA prefill overwrites
+//           ring slots the prefix reads: then it runs first, in a launch of its own.
 //  flash:   one workgroup per (32-position query block, kv head) serves the 8 q
 //           heads of the group (256 query rows, 8 waves x 1 head x 32 rows), so
 //           a K/V tile is staged in LDS once per 256 rows. Q is normalised,
@@ -96,16 +96,18 @@ __device__ inline void put_texp(const PrefillParams &P, int kvh, int row0, int e
 // grid (tiles, kv head), 256 threads. Block x takes tile n_direct + x; a whole tile of cached positions: a
 // cache tile and a copy tile both hold 16-byte units of 8 dims of one key (K) or 8 keys of one
 // dim (V), so each thread moves 2 + 2 units: read, measure, scale, convert to f16, write at
-// the unit's place in the copy. When p0 is not 32-aligned, one more block copies the cached
-// positions [p0 & ~31, p0) of the tile that holds p0 into their places in the copy as the
+// the unit's place in the copy. In a launch of its own, when p0 is not 32-aligned, one more block copies the
+// cached positions [p0 & ~31, p0) of the tile that holds p0 into their places in the copy as the
 // cache's raw 16-bit values: kv_prep takes them from there (a long SWA prefill overwrites
 // their ring slots in its own launch) and writes the tile, new positions included.
+// Every other call runs it as blocks behind kv_prep's chunks: the two are mostly latency, 3-5 us each. Two
+// launches -> one, the whole call: 10 tokens at 1500 cached (full, f16) 26.2 -> 22.7 us, 30 at 5000 (SWA,
+// bf16) 26.0 -> 23.4, 1000 at 7000 (full, bf16) 169.3 -> 165.6.
 template <int DT>
-__global__ __launch_bounds__(256) void prefix_kernel(const PrefillParams P) {
+__device__ inline void prefix_tile(const PrefillParams &P, int tile, int kvh, float (&red)[2][4]) {
     typedef KvType<DT> KT;
-    __shared__ float red[2][4];
-    const int kvh = blockIdx.y, tid = threadIdx.x;
-    const int row0 = 32 * (P.n_direct + (int)blockIdx.x), pos0 = P.kbase + row0;  // the tile's first position
+    const int tid = threadIdx.x;
+    const int row0 = 32 * (P.n_direct + tile), pos0 = P.kbase + row0;  // the tile's first position
     const int crow = row0 - 32 * P.n_direct;  // its row in the copy, which starts at tile n_direct
     if (pos0 + 32 > P.p0) {  // the tile holding p0: raw values of positions [pos0, p0)
         // every load before the first store: a load after a store that may alias it (both
@@ -168,6 +170,11 @@ __global__ __launch_bounds__(256) void prefix_kernel(const PrefillParams P) {
         *(f16x8 *)(P.sk + pv_index(kvh, crow + 8 * (u & 3), u >> 2, P.k_rows)) = v8;
     }
 }
+template <int DT>
+__global__ __launch_bounds__(256) void prefix_kernel(const PrefillParams P) {
+    __shared__ float red[2][4];
+    prefix_tile<DT>(P, blockIdx.x, blockIdx.y, red);
+}
 
 // ---------------------------------------------------------------------------
 // kv_prep: the new tokens' K and V. grid (32-position chunks, kv head), 4 waves.
@@ -180,8 +187,8 @@ __global__ __launch_bounds__(256) void prefix_kernel(const PrefillParams P) {
 // K units (one key, 8 dims) and V units (one dim, these 8 keys), scaled by the tile's
 // exponents, and the cache's units of the new positions it keeps. So an f16 chunk needs no
 // workgroup barrier (a bf16 chunk has one, for the tile's exponents). The first chunk also
-// takes the cached positions before p0 (from the copy, where prefix_kernel left their raw
-// values), and rows past the last new position are zero. A V unit of the cache spans the 8
+// takes the cached positions before p0 (from the cache, or from the copy where prefix_kernel left their
+// raw values), and rows past the last new position are zero. A V unit of the cache spans the 8
 // positions: where some of them are not new (or, for the ring, not kept) its elements are
 // stored one by one, so no cache unit is read back and no two workgroups write the same bytes.
 constexpr int KP_WAVES = 4, KP_THREADS = 64 * KP_WAVES, KP_ROWS = 32 / KP_WAVES;  // rows per wave
@@ -194,6 +201,11 @@ __global__ __launch_bounds__(KP_THREADS) void kv_prep_kernel(const PrefillParams
     __shared__ float red[2][KP_WAVES];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kvh = blockIdx.y;
+    const int n_chunks = ((P.p0 + P.T + 31) >> 5) - (P.p0 >> 5);
+    if ((int)blockIdx.x >= n_chunks) {  // one launch: a whole tile of cached positions
+        prefix_tile<DT>(P, blockIdx.x - n_chunks, kvh, red);
+        return;
+    }
     const int c0 = (P.p0 >> 5) + blockIdx.x, pos0 = 32 * c0;  // first position of the chunk
     const int lo = max(P.p0, pos0), hi = min(P.p0 + P.T, pos0 + 32);  // new positions [lo, hi)
     const int r0 = KP_ROWS * wave;  // this wave's rows r0 .. r0 + 7
@@ -213,6 +225,27 @@ __global__ __launch_bounds__(KP_THREADS) void kv_prep_kernel(const PrefillParams
     for (int k = 0; k < 4; k++) kx[k] = *(const float4 *)(kr + 32 * k);
 #pragma unroll
     for (int k = 0; k < 4; k++) vx[k] = *(const float4 *)(kr + KV_DIM + 32 * k);
+    // the first chunk of a continuation that starts inside a tile: its cached positions [pos0, p0), from
+    // the cache, or from the copy, where prefix_kernel left the cache's raw values (kbase <= pos0,
+    // 32-aligned). All rows' loads together (rows from lo on re-read the first row), so they share
+    // one round trip
+    const bool has_cached = pos0 + r0 < lo;  // wave-uniform
+    uint16_t rk[KP_ROWS][2], rv[KP_ROWS][2];
+    if (has_cached) {
+        const uint16_t *const raw_k = P.one_launch ? P.cache_k : (const uint16_t *)P.sk;
+        const uint16_t *const raw_v = P.one_launch ? P.cache_v : (const uint16_t *)P.sk;
+        const int slot0 = pos0 & P.cache_mask, row0 = pos0 - P.kbase - 32 * P.n_direct;  // the copy starts at tile n_direct
+#pragma unroll
+        for (int i = 0; i < KP_ROWS; i++) {
+            const int r = pos0 + r0 + i < lo ? r0 + i : r0;
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                const int d = lane + 64 * h;
+                rk[i][h] = raw_k[P.one_launch ? kt_index(kvh, slot0 + r, d, P.n_slots) : pk_index(kvh, row0 + r, d, P.k_rows)];
+                rv[i][h] = raw_v[P.one_launch ? vt_index(kvh, slot0 + r, d, P.n_slots) : pv_index(kvh, row0 + r, d, P.k_rows)];
+            }
+        }
+    }
     float ss = 0.f;
 #pragma unroll
     for (int k = 0; k < 4; k++) ss += kx[k].x * kx[k].x + kx[k].y * kx[k].y + kx[k].z * kx[k].z + kx[k].w * kx[k].w;
@@ -256,20 +289,7 @@ __global__ __launch_bounds__(KP_THREADS) void kv_prep_kernel(const PrefillParams
         }
         *(uint2 *)&kl[r][32 * k + 4 * q8] = make_uint2(pack2(kh[0], kh[1]), pack2(kh[2], kh[3]));
     }
-    if (pos0 + r0 < lo) {  // wave-uniform
-        // the first chunk of a continuation that starts inside a tile: its cached positions
-        // [pos0, p0) come from the copy, where prefix_kernel left the cache's raw values
-        // (kbase <= pos0, 32-aligned)
-        const uint16_t *raw = (const uint16_t *)P.sk;
-        // all rows' loads first (rows from lo on re-read the first row), so they share one round trip
-        uint16_t rk[KP_ROWS][2], rv[KP_ROWS][2];
-#pragma unroll
-        for (int i = 0; i < KP_ROWS; i++) {
-            const int r = pos0 + r0 + i < lo ? r0 + i : r0;
-            const int row = pos0 + r - P.kbase - 32 * P.n_direct;  // the copy starts at tile n_direct
-            rk[i][0] = raw[pk_index(kvh, row, lane, P.k_rows)], rk[i][1] = raw[pk_index(kvh, row, lane + 64, P.k_rows)];
-            rv[i][0] = raw[pv_index(kvh, row, lane, P.k_rows)], rv[i][1] = raw[pv_index(kvh, row, lane + 64, P.k_rows)];
-        }
+    if (has_cached) {
 #pragma unroll
         for (int i = 0; i < KP_ROWS; i++) {
             const int r = r0 + i;
@@ -876,15 +896,18 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(const PrefillParam
 }
 
 hipError_t launch_prefill(const PrefillParams &P, int dtype, hipStream_t stream) {
-    // tiles holding cached positions (kbase 32-aligned) that the copy takes from the cache
-    const int n_pre = ((P.p0 - P.kbase + 31) >> 5) - P.n_direct;
+    // tiles holding cached positions (kbase 32-aligned) that the copy takes from the cache; in one launch
+    // kv_prep's first chunk takes those of the tile that holds p0 itself
+    const int n_chunks = ((P.p0 + P.T + 31) >> 5) - (P.p0 >> 5);
+    const int n_pre = ((P.p0 - P.kbase + (P.one_launch ? 0 : 31)) >> 5) - P.n_direct;
     const int nqb = (P.T + PF_BQ - 1) / PF_BQ;
-    const dim3 gp(n_pre, N_HEAD_KV), gk(((P.p0 + P.T + 31) >> 5) - (P.p0 >> 5), N_HEAD_KV);
+    const dim3 gp(n_pre, N_HEAD_KV), gk(n_chunks + (P.one_launch ? n_pre : 0), N_HEAD_KV);
+    const bool prefix = n_pre > 0 && !P.one_launch;
     if (dtype == DT_F16) {
-        if (n_pre > 0) hipLaunchKernelGGL(prefix_kernel<DT_F16>, gp, dim3(256), 0, stream, P);
+        if (prefix) hipLaunchKernelGGL(prefix_kernel<DT_F16>, gp, dim3(256), 0, stream, P);
         hipLaunchKernelGGL(kv_prep_kernel<DT_F16>, gk, dim3(KP_THREADS), 0, stream, P);
     } else {
-        if (n_pre > 0) hipLaunchKernelGGL(prefix_kernel<DT_BF16>, gp, dim3(256), 0, stream, P);
+        if (prefix) hipLaunchKernelGGL(prefix_kernel<DT_BF16>, gp, dim3(256), 0, stream, P);
         hipLaunchKernelGGL(kv_prep_kernel<DT_BF16>, gk, dim3(KP_THREADS), 0, stream, P);
     }
     if (P.n_direct > 0)

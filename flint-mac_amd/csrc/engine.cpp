@@ -276,6 +276,10 @@ void prefill_impl(const flint_attn_layer *L, const float *qkv, int q_stride, int
     // window (masked keys).
     if (L->kv_dtype == FLINT_KV_F16 && T <= 256 && (!L->is_swa || T <= L->n_slots - L->window + 1))
         P.n_direct = (p0 - P.kbase) >> 5;
+    // the new positions' slots last held positions below p0 + T - n_slots: with those before kbase, the cached
+    // positions are converted in kv_prep's launch (always on full layers, and for T <= n_slots - window - 30
+    // on a ring)
+    P.one_launch = p0 + T - L->n_slots <= P.kbase;
     // the attention copy holds the positions from tile n_direct on, then its table of per-tile
     // exponents (every tile the flash kernel reads from it is written in this call, padding
     // rows included): a short call at a long context needs only its own few tiles

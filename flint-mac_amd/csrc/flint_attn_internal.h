@@ -77,6 +77,9 @@ struct PrefillParams {
     // caches, where the copy would hold the same bits, when no cache slot they read is rewritten
     // by this call's kv_prep with a key some query still needs; 0 otherwise
     int n_direct;
+    // kv_prep's launch also converts the cached positions: no slot that it writes holds one of
+    // [kbase, p0); 0: prefix_kernel has run before it
+    int one_launch;
     unsigned call_id;     // nonzero id of this call (see g_scaled_call in attn_prefill.hip)
     float *att;           // [T][4096]
     // key splits (few query blocks over a long key range): each query block's tiles in n_split

@@ -384,6 +384,36 @@ def test_prefill_blocks_whole_and_split(cuda, store, T, p0):
     assert_close(att.cpu().numpy(), want, f"T={T} p0={p0} {store}")
 
 
+@pytest.mark.parametrize("store", ["f16", "bf16"])
+@pytest.mark.parametrize("is_swa,T,p0", [(True, 501, 1003), (True, 502, 1003), (True, 480, 1023), (True, 511, 992), (True, 3, 2078),
+                                         (False, 1, 1023), (False, 66, 959)])
+def test_prefill_cached_positions_with_the_new_ones(cuda, store, is_swa, T, p0):
+    """Continuations whose cached positions are converted in the launch that writes the new ones, up to the
+    longest that leaves their ring slots alone (p0 = 1003 reads slots from position 480 on: 501 tokens; p0 =
+    992 and 1023, 512 and 513) and one more: outputs and the whole ring against the oracle."""
+    rng = np.random.default_rng(T + p0)
+    qn, kn, sk = layer_weights(rng)
+    n = p0 + T
+    kv = fa.KVLayer(is_swa=is_swa, has_rope=True, n_slots=1024 if is_swa else (n + 31) // 32 * 32, kv_dtype=store,
+                    rope_theta=1e4, q_norm=qn, k_norm=kn, sinks=sk)
+    L = oracle_layer(kv, qn, kn, sk, store)
+    qkv = rng.standard_normal((n, QKV_DIM)).astype(np.float32)
+    dq = torch.from_numpy(qkv).to(cuda)
+    att = torch.full((n, Q_DIM), float("nan"), device=cuda)
+    kv.prefill(dq[:p0], att[:p0], 0)
+    kv.prefill(dq[p0:], att[p0:], p0)
+    torch.cuda.synchronize()
+    K = np.zeros((n, KV_DIM), np.float32)
+    V = np.zeros((n, KV_DIM), np.float32)
+    want = fo.prefill(L, qkv, 0, K, V, n_threads=16)
+    assert_close(att[p0:].cpu().numpy(), want[p0:], f"T={T} p0={p0} {store}")
+    vc, kc = kv.v_slots()[0].float().cpu().numpy(), kv.k_slots()[0].float().cpu().numpy()
+    pos = np.arange(n - 1024 if is_swa else 0, n)
+    s = pos & 1023 if is_swa else pos
+    assert np.array_equal(vc[:, s], V[pos].reshape(-1, N_HEAD_KV, HEAD_DIM).transpose(1, 0, 2))
+    assert k_close(kc[:, s], K[pos].reshape(-1, N_HEAD_KV, HEAD_DIM).transpose(1, 0, 2), store)
+
+
 @pytest.mark.parametrize("is_swa", [False, True], ids=["full", "swa"])
 def test_prefill_f16_cached_tiles_on_scaled_path(cuda, is_swa):
     """An f16 continuation reads its whole cached tiles from the cache itself; with q gains
