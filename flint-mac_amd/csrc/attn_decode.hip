@@ -45,6 +45,7 @@
 //    are packed so that a kv head's slices share one XCD: its K comes from HBM once and
 //    from that XCD's L2 for the other slices.
 #include <mutex>
+#include <type_traits>
 
 #include "common.h"
 #include "flint_attn_internal.h"
@@ -184,8 +185,25 @@ __device__ inline void consume_tile(DecodeState<DT, VS> &S, KvTile<VS> &T, const
     for (int d = 0; d < 8 / VS; d++) S.acc[d] = KT::mfma16(__builtin_bit_cast(typename KT::vec8, T.v[d]), pb, S.acc[d]);
 }
 
-template <int DT, int VS>
-__global__ __launch_bounds__(DEC_THREADS) void attn_decode_kernel(const DecodeParams P) {
+// What a launch for one sequence reads beyond its plain arguments.
+struct DecodeOne {
+    const float *k_norm, *sinks;
+    float *att, *partial;
+    float rope_freq[64];
+};
+
+// The plain arguments (14 words, preloaded into SGPRs) are what a wave needs to request its first tile.
+// shape = is_swa | has_rope << 1 | n_split << 2. ONE: one sequence, whose position and plan are plain arguments
+// (pos, tps, n_split); otherwise the sequences' tables are in P and these are unused. With every argument in a
+// struct, whose round trip and tables' loads came first: one SWA layer (513 keys) 5.48 us, now 5.24; a full
+// layer at 6000 keys with the merge 10.1 and 9.2, at 32768 14.9 and 14.1; a step of Flint's 49 layers at
+// 6001 tokens 831 and 798. Batches are as they were (5 sequences 6.0-6.1 us).
+template <int DT, int VS, bool ONE>
+__global__ __launch_bounds__(DEC_THREADS) void attn_decode_kernel(const float *qkv, uint16_t *k_cache, uint16_t *v_cache,
+                                                                  const float *q_norm, const int pos1, const int tps1,
+                                                                  const int n_slots, const int shape, const int window,
+                                                                  const float rms_eps,
+                                                                  const std::conditional_t<ONE, DecodeOne, DecodeParams> P) {
     typedef KvType<DT> KT;
     typedef typename KT::vec8 vec8;
     constexpr int W = DEC_WAVES;
@@ -196,25 +214,23 @@ __global__ __launch_bounds__(DEC_THREADS) void attn_decode_kernel(const DecodePa
     const int hloc = n & 7, hl = n >> 3;      // head within the GQA group, 0 = hi half, 1 = lo half
     static_assert(MAX_SEQ == 64, "one per-sequence table entry per lane");
 
-    // ---- every kernel argument is read here, in one batch of loads at wave start (left to
-    //      itself the compiler sinks each load to its first use, and each sunk load is one
-    //      more memory round trip on the critical path). The per-sequence tables arrive one
-    //      entry per lane, so finding this workgroup's sequence costs no second round trip ----
-    const int t_base = P.wg_base[lane], t_pos = P.pos[lane], t_tps = P.tps[lane], t_ns = P.n_split[lane];
-    const int t_s0 = P.split0[lane];
-    const int n_seq = P.n_seq;
-    const int is_swa = P.is_swa, has_rope = P.has_rope, window = P.window;
-    const int n_slots = P.n_slots, slot_mask = P.slot_mask;
-    const float rms_eps = P.rms_eps;
-    const long long seq_stride = P.seq_stride;
-    const float *const qkv = P.qkv, *const q_norm = P.q_norm, *const k_norm = P.k_norm, *const sinks = P.sinks;
-    uint16_t *const k_cache = P.k_cache, *const v_cache = P.v_cache;
-    float *const att = P.att, *const partial = P.partial;
-    pin_sgpr(n_seq), pin_sgpr(is_swa), pin_sgpr(has_rope), pin_sgpr(window);
-    pin_sgpr(n_slots), pin_sgpr(slot_mask), pin_sgpr(rms_eps), pin_sgpr(seq_stride);
-    pin_sgpr(qkv), pin_sgpr(q_norm), pin_sgpr(k_norm), pin_sgpr(sinks), pin_sgpr(k_cache), pin_sgpr(v_cache);
-    pin_sgpr(att), pin_sgpr(partial);
-    asm volatile("" ::"v"(t_base), "v"(t_pos), "v"(t_tps), "v"(t_ns), "v"(t_s0));
+    const int is_swa = shape & 1, has_rope = shape & 2, slot_mask = is_swa ? n_slots - 1 : 0x7fffffff;
+    int n_seq = 1, t_base = 0, t_pos = 0, t_tps = 0, t_ns = 0, t_s0 = 0;
+    long long seq_stride = 0;
+    const float *k_norm = P.k_norm, *sinks = P.sinks;
+    float *att = P.att, *partial = P.partial;
+    if constexpr (!ONE) {
+        // ---- every other argument is read here, in one batch of loads at wave start (left to
+        //      itself the compiler sinks each load to its first use, and each sunk load is one
+        //      more memory round trip on the critical path). The per-sequence tables arrive one
+        //      entry per lane, so finding this workgroup's sequence costs no second round trip ----
+        t_base = P.wg_base[lane], t_pos = P.pos[lane], t_tps = P.tps[lane], t_ns = P.n_split[lane];
+        t_s0 = P.split0[lane];
+        n_seq = P.n_seq, seq_stride = P.seq_stride;
+        pin_sgpr(n_seq), pin_sgpr(seq_stride);
+        pin_sgpr(k_norm), pin_sgpr(sinks), pin_sgpr(att), pin_sgpr(partial);
+        asm volatile("" ::"v"(t_base), "v"(t_pos), "v"(t_tps), "v"(t_ns), "v"(t_s0));
+    }
 
     // The grid is flat and holds exactly the launch's work units: sequence s owns workgroups
     // wg_base[s] .. wg_base[s] + 4 VS n_split[s] - 1 (kv head fastest, then V slice, then
@@ -232,11 +248,14 @@ __global__ __launch_bounds__(DEC_THREADS) void attn_decode_kernel(const DecodePa
         if (s >= n_seq) return;  // the second sequence of the last block when n_seq is odd
         wid = 4 * VS * s + (j & 3) + 4 * (j >> 3);  // kv head j & 3, V slice j >> 3
     }
-    const int seq = __builtin_popcountll(__builtin_amdgcn_ballot_w64(lane < n_seq && wid >= t_base)) - 1;
-    const int n_split = __builtin_amdgcn_readlane(t_ns, seq), pos = __builtin_amdgcn_readlane(t_pos, seq);
-    const int tps = __builtin_amdgcn_readlane(t_tps, seq);
-    const int local = wid - __builtin_amdgcn_readlane(t_base, seq);
-    const int split0 = __builtin_amdgcn_readlane(t_s0, seq);  // this sequence's first partial record
+    int seq = 0, n_split = shape >> 2, pos = pos1, tps = tps1, local = wid, split0 = 0;
+    if constexpr (!ONE) {
+        seq = __builtin_popcountll(__builtin_amdgcn_ballot_w64(lane < n_seq && wid >= t_base)) - 1;
+        n_split = __builtin_amdgcn_readlane(t_ns, seq), pos = __builtin_amdgcn_readlane(t_pos, seq);
+        tps = __builtin_amdgcn_readlane(t_tps, seq);
+        local = wid - __builtin_amdgcn_readlane(t_base, seq);
+        split0 = __builtin_amdgcn_readlane(t_s0, seq);  // this sequence's first partial record
+    }
     const int kvh = local & (N_HEAD_KV - 1), slice = (local / N_HEAD_KV) % VS, split = local / (N_HEAD_KV * VS);
     if (seq < 0 || split >= n_split) return;  // not reached: the host sizes the grid exactly
     const bool last_split = split == n_split - 1;
@@ -265,11 +284,6 @@ __global__ __launch_bounds__(DEC_THREADS) void attn_decode_kernel(const DecodePa
     const float2 qx = make_float2(qr[lane], qr[lane + 64]);
     const float2 qw = make_float2(q_norm[lane], q_norm[lane + 64]);
     const float rfreq = P.rope_freq[lane];
-    // head `wave` of the group, for the final merge: a wave-uniform address read through the
-    // constant address space, so it is a scalar load into an SGPR that nothing waits for until
-    // the merge (the kernel never writes the sinks). A vector load moved into an SGPR here made
-    // every wave wait for its round trip before it issued its first tile loads.
-    const float sink = *(const __attribute__((address_space(4))) float *)(sinks + kvh * GQA + wave) * LOG2E;
     float2 kx = {0.f, 0.f}, kw = {0.f, 0.f}, vx = {0.f, 0.f};
     if (cur_wave) {
         const float *kr = row + Q_DIM + kvh * HEAD_DIM, *vr = row + Q_DIM + KV_DIM + kvh * HEAD_DIM;
@@ -291,6 +305,12 @@ __global__ __launch_bounds__(DEC_THREADS) void attn_decode_kernel(const DecodePa
     int t_a = t_begin + wave, t_b = t_a + W;
     load_tile(ta, kc, vc, t_a < t_end ? t_a : t_begin, lane, slot_mask, t_a < t_end, slice);
     __builtin_amdgcn_sched_barrier(0);
+    if constexpr (ONE) pin_sgpr(sinks), pin_sgpr(att), pin_sgpr(partial);  // waited for here, behind the tile's loads
+    // head `wave` of the group, for the final merge: a wave-uniform address read through the
+    // constant address space, so it is a scalar load into an SGPR that nothing waits for until
+    // the merge (the kernel never writes the sinks). A vector load moved into an SGPR here made
+    // every wave wait for its round trip.
+    const float sink = *(const __attribute__((address_space(4))) float *)(sinks + kvh * GQA + wave) * LOG2E;
     // The current token's rows are handed to the prologue here, after the tile's loads: left
     // alone, the compiler rounds v to the cache dtype right after its load, in the branch
     // above, and that wave then waits for the load before it issues its tile.
@@ -444,11 +464,9 @@ __global__ __launch_bounds__(DEC_THREADS) void attn_decode_kernel(const DecodePa
     if (lane2 == 0) *(float2 *)(pp + HEAD_DIM) = make_float2(M, L);
 }
 
-// The merge kernel's arguments: only what it reads (536 bytes instead of the decode kernel's
-// 1.3 KB), since a dependent launch waits for its argument block.
+// The merge kernel's tables for several sequences: only what it reads (512 bytes instead of the decode
+// kernel's 1.9 KB), since a dependent launch waits for its argument block.
 struct CombineParams {
-    const float *partial, *sinks;
-    float *att;
     int n_split[MAX_SEQ];  // key splits of sequence s
     int split0[MAX_SEQ];   // first split record of sequence s
 };
@@ -468,13 +486,12 @@ __device__ inline float dpp_half_mirror(float x) {
 // At most 2 waves per SIMD (one workgroup per CU is all the grid needs), so the register
 // allocator keeps a lane's 8 accumulator loads and its (m, l) load in flight together instead
 // of reusing registers for the last loads after a wait (a second memory round trip).
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void attn_combine_kernel(const CombineParams P) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void attn_combine_kernel(
+    const float *partial, const float *sinks, float *att, const int ns1, const CombineParams P) {
     const int hh = blockIdx.x, seq = blockIdx.y, lane = threadIdx.x & 63;
     const int q = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int ns = P.n_split[seq], split0 = P.split0[seq];
-    const float *const partial = P.partial, *const sinks = P.sinks;
-    float *const att = P.att;
-    pin_sgpr(ns), pin_sgpr(split0), pin_sgpr(partial), pin_sgpr(sinks), pin_sgpr(att);
+    int ns = ns1, split0 = 0;  // one sequence's splits, a preloaded argument like the pointers; 0: tables
+    if (ns1 == 0) ns = P.n_split[seq], split0 = P.split0[seq];
     if (ns <= 1) return;  // written directly by the decode kernel
     const float *pp = partial + ((size_t)split0 * N_HEAD + hh * ns) * PART_STRIDE;
     // a scalar load (constant address space: the kernel never writes the sinks), first used
@@ -558,38 +575,41 @@ hipError_t decode_scratch(float **ptr) {
     return hipSuccess;
 }
 
+template <int DT, int VS>
+static void launch_decode_vs(const DecodeParams &P, dim3 grid, hipStream_t stream) {
+    const int shape = (P.is_swa ? 1 : 0) | (P.has_rope ? 2 : 0) | P.n_split[0] << 2;
+    if constexpr (VS == 1 || VS == 8)
+        if (P.n_seq == 1) {
+            DecodeOne one{P.k_norm, P.sinks, P.att, P.partial, {}};
+            for (int i = 0; i < HEAD_DIM / 2; i++) one.rope_freq[i] = P.rope_freq[i];
+            hipLaunchKernelGGL((attn_decode_kernel<DT, VS, true>), grid, dim3(DEC_THREADS), 0, stream, P.qkv, P.k_cache, P.v_cache,
+                               P.q_norm, P.pos[0], P.tps[0], P.n_slots, shape, P.window, P.rms_eps, one);
+            return;
+        }
+    hipLaunchKernelGGL((attn_decode_kernel<DT, VS, false>), grid, dim3(DEC_THREADS), 0, stream, P.qkv, P.k_cache, P.v_cache,
+                       P.q_norm, 0, 0, P.n_slots, shape, P.window, P.rms_eps, P);
+}
+
 hipError_t launch_decode(const DecodeParams &P, int dtype, hipStream_t stream) {
     // V slices: ids packed by XCD, 8 VS per pair of sequences (the kernel maps them back)
-    const int n_wg = P.v_slices > 1 ? 8 * P.v_slices * ((P.n_seq + 1) / 2) : P.wg_base[P.n_seq];
-    dim3 grid(n_wg), block(DEC_THREADS);
-    if (dtype == DT_F16 && P.v_slices == 8)
-        hipLaunchKernelGGL((attn_decode_kernel<DT_F16, 8>), grid, block, 0, stream, P);
-    else if (dtype == DT_BF16 && P.v_slices == 8)
-        hipLaunchKernelGGL((attn_decode_kernel<DT_BF16, 8>), grid, block, 0, stream, P);
-    else if (dtype == DT_F16 && P.v_slices == 4)
-        hipLaunchKernelGGL((attn_decode_kernel<DT_F16, 4>), grid, block, 0, stream, P);
-    else if (dtype == DT_BF16 && P.v_slices == 4)
-        hipLaunchKernelGGL((attn_decode_kernel<DT_BF16, 4>), grid, block, 0, stream, P);
-    else if (dtype == DT_F16 && P.v_slices == 2)
-        hipLaunchKernelGGL((attn_decode_kernel<DT_F16, 2>), grid, block, 0, stream, P);
-    else if (dtype == DT_F16)
-        hipLaunchKernelGGL((attn_decode_kernel<DT_F16, 1>), grid, block, 0, stream, P);
-    else if (P.v_slices == 2)
-        hipLaunchKernelGGL((attn_decode_kernel<DT_BF16, 2>), grid, block, 0, stream, P);
-    else
-        hipLaunchKernelGGL((attn_decode_kernel<DT_BF16, 1>), grid, block, 0, stream, P);
+    const dim3 grid(P.v_slices > 1 ? 8 * P.v_slices * ((P.n_seq + 1) / 2) : P.wg_base[P.n_seq]);
+    const bool f16 = dtype == DT_F16;
+    switch (P.v_slices) {
+        case 8: f16 ? launch_decode_vs<DT_F16, 8>(P, grid, stream) : launch_decode_vs<DT_BF16, 8>(P, grid, stream); break;
+        case 4: f16 ? launch_decode_vs<DT_F16, 4>(P, grid, stream) : launch_decode_vs<DT_BF16, 4>(P, grid, stream); break;
+        case 2: f16 ? launch_decode_vs<DT_F16, 2>(P, grid, stream) : launch_decode_vs<DT_BF16, 2>(P, grid, stream); break;
+        default: f16 ? launch_decode_vs<DT_F16, 1>(P, grid, stream) : launch_decode_vs<DT_BF16, 1>(P, grid, stream);
+    }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     if (P.max_split > 1) {
         CombineParams C;
-        C.partial = P.partial;
-        C.sinks = P.sinks;
-        C.att = P.att;
         for (int s = 0; s < MAX_SEQ; s++) {
             C.n_split[s] = s < P.n_seq ? P.n_split[s] : 0;
             C.split0[s] = s < P.n_seq ? P.split0[s] : 0;
         }
-        hipLaunchKernelGGL(attn_combine_kernel, dim3(N_HEAD, P.n_seq), dim3(256), 0, stream, C);
+        hipLaunchKernelGGL(attn_combine_kernel, dim3(N_HEAD, P.n_seq), dim3(256), 0, stream, P.partial, P.sinks, P.att,
+                           P.n_seq == 1 ? P.n_split[0] : 0, C);
         e = hipGetLastError();
     }
     return e;
