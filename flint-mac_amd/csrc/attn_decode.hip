@@ -37,9 +37,9 @@
 //  * Batched entry: one launch serves many independent sequences (one token each).
 //    The grid is flat: sequence s owns 4 x n_split[s] consecutive workgroups (kv head
 //    fastest), so no workgroup is idle and the XCDs, dealt workgroups in id order, get
-//    equal shares of the stream. Every kernel argument the block needs is read at wave
-//    start (the per-sequence tables one entry per lane), so the kernel-argument fetch
-//    costs one memory round trip.
+//    equal shares of the stream. What a wave needs for its first tile is preloaded into SGPRs; a
+//    batch's other arguments are read at wave start (the per-sequence tables one entry per
+//    lane), so their fetch costs one memory round trip.
 //  * Short key ranges (one split per sequence, SWA layers): a kv head's 128 output dims
 //    are cut over 8 (4, 2) V-slice workgroups, each reading all of K, and the launch ids
 //    are packed so that a kv head's slices share one XCD: its K comes from HBM once and

@@ -88,16 +88,17 @@ int32_t flint_attn_o_proj(const flint_weight *wo, const float *att, float *x, vo
  * The same two projections for n_tok tokens (the prefill side):
  * x: device [n_tok][2048]; qkv: device [n_tok] rows of qkv_stride floats (>= 5120), the raw
  * q|k|v at each row's start; att: device [n_tok][4096].
- * Below 16 tokens (or when the output rows are not 16-byte aligned) each token runs the
- * single-token kernel and gets exactly its bits. From 16 tokens the batch runs as a GEMM on
+ * Below 16 tokens (or when the output rows are not 16-byte aligned) each token gets exactly the
+ * bits of its single-token call. From 16 tokens the batch runs as a GEMM on
  * the matrix cores: weight and activation rows split into f16 hi/lo pairs (22 bits, each row
  * scaled by a power of two), products summed in fp32 (q8_0, iq4_xs, q5_K and q6_K weights keep
  * their integer values, exact in f16, and take their block scales and mins in fp32; f16
  * weights are used as they are, bf16 ones scaled by a power of two per block of 32); every
  * output is within fp32 reassociation of the single-token result (both within the oracle's
- * bound). Batches run in passes of at most 8192 tokens, so the device workspace has a ceiling:
- * 4 (rows + p) x K bytes, p = the pass's tokens padded to 128 (and p K / 8 more with q5_K
- * weights), allocated on first use and reused.
+ * bound). Up to 480 tokens (no f32 weights) the GEMM reads the GGUF rows themselves, above that it
+ * builds weight planes first. Batches run in passes of at most 8192 tokens, so the device workspace
+ * has a ceiling: 4 (rows + p) x K bytes, p = the pass's tokens padded to 128 (and p K / 8 more with
+ * q5_K weights), allocated on first use and reused.
  * Replace the prefill's k_rmsnorm_rows + three mm (q, k, v), and mm(o) + k_add_rows, at
  * /root/reference/src/engine.mm:1083-1086 and 1105-1111.
  */
