@@ -172,7 +172,6 @@ void decode_impl(const flint_attn_layer *L, int n_seq, int64_t seq_stride, const
     P.seq_stride = seq_stride;
     P.att = att;
     P.n_slots = L->n_slots;
-    P.slot_mask = L->is_swa ? L->n_slots - 1 : 0x7fffffff;
     P.is_swa = L->is_swa;
     P.has_rope = L->has_rope;
     P.window = L->window;

@@ -25,8 +25,7 @@ struct DecodeParams {
     float *att;                 // [n_seq][4096]
     float *partial;             // [sum of n_split over sequences of more than one split][32][132]:
                                 // sequence s's records start at split0[s], each head's consecutive
-    int n_slots;                // slots per kv head
-    int slot_mask;              // SWA: n_slots - 1 (power of two); full: all ones
+    int n_slots;                // slots per kv head (SWA: a power of two, slot = position & (n_slots - 1))
     int is_swa, has_rope, window, max_split;
     float rms_eps;
     int n_seq;
