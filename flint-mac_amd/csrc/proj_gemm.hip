@@ -725,6 +725,7 @@ __global__ __launch_bounds__(GM_THREADS, EU) void gemm_int_kernel(const GemmPara
     constexpr int SCB = gq_scales<SUB>(), SCL = SCB / 16;  // scales per chunk; lanes that load them
     constexpr int STAGE = gq_stage<SUB, TB>(), LOADS = 2 * TB + 2 + 1 + (MIN ? 2 : 0);  // direct loads per wave per chunk
     constexpr int TT = 64 * TB, XP = TT * GM_KC * 2;  // tokens; bytes of an x plane's chunk
+    static_assert(LOADS * (STAGES - 1) < 64, "the loads in flight fit vmcnt");
     __shared__ __align__(16) uint8_t lds[STAGES][gq_bytes<SUB, MIN, TB>()];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -847,12 +848,13 @@ __global__ __launch_bounds__(GM_THREADS, EU) void gemm_int_kernel(const GemmPara
     // last chunk it re-reads the last one into a stage no one reads again), so "chunk c has
     // landed" is vmcnt(LOADS (STAGES - 2)) with the chunks after it still in flight; the barrier then
     // makes every wave's part of it visible, and it also ends every wave's reads of the stage of chunk
-    // c - 1, which chunk c + STAGES - 1 overwrites after it. No fence: a workgroup-scope fence would
-    // wait for every load in flight (vmcnt(0)); the empty asm keeps the compiler from moving LDS reads
-    // across the barrier, and the chunk before's reads have all returned (their registers fed its MFMAs).
+    // c - 1, which chunk c + STAGES - 1 overwrites after it. Those reads are waited for too: the ones that feed
+    // FMAs (scales, token sums, mins) are otherwise still on their way here, since the FMAs that use them
+    // follow the barrier. The wait is asm with a memory clobber, so that no LDS access moves past it
+    // or across the barrier. No fence: a workgroup-scope fence would wait for every load in flight (vmcnt(0)).
     int st = 0;
     auto sync = [&](int c) {
-        wait_vmcnt<LOADS *(STAGES - 2)>();
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(LOADS *(STAGES - 2)) : "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
         const int at = st;
