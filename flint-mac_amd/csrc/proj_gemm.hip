@@ -306,7 +306,7 @@ struct RawCopy {
             if (NU % 64 == 0 || i < WL - 1 || 64 * i + lane < NU) *(u32x4 *)(area + lo[i]) = w[i];
     }
 };
-__device__ inline void wave_lds_fence() {  // the wave's LDS stores before its LDS loads
+__device__ inline void wave_lds_fence() {  // the wave's LDS accesses so far stay ahead of those to come
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -1001,6 +1001,7 @@ __device__ __forceinline__ void gemm_raw_segment(const GemmParams &P, const uint
     for (int c = 0; c < GR_CHUNKS; c++) {
         const int q = c / G, j = c % G;
         if (j == 0) {
+            if (q > 0) wave_lds_fence();  // the group before's reads, of other types, stay ahead of these stores
             C.store(area, lane);
             if (MIN && q == 0) *(f32x4 *)(sums + 16 * lane) = S0, *(f32x4 *)(sums + 1024 + 16 * lane) = S1;
             wave_lds_fence();
