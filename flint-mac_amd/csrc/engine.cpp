@@ -401,8 +401,7 @@ void proj_gemm(const MatvecSeg *seg, int n_seg, int N, int K, const float *x, lo
                float eps, int T, float *y, long long y_stride, int add, const WeightPlanes *pl, hipStream_t stream,
                bool build_only = false) {
     const IntForm form = gemm_int_form(seg, n_seg);
-    // short batches in the integer form read the GGUF rows themselves: no weight planes
-    const bool raw = form.sub && !build_only && T <= (pl ? GEMM_RAW_TOKENS_KEPT : GEMM_RAW_TOKENS);
+    const bool raw = !build_only && !gemm_reads_planes(form, T, pl != nullptr);
     const int T_pass = build_only ? 0 : std::min(T, GEMM_PASS_TOKENS);
     const int T_pad = (T_pass + GEMM_TILE - 1) / GEMM_TILE * GEMM_TILE;
     const size_t wbytes = pl || raw ? 0 : (size_t)N * K * sizeof(_Float16), xbytes = (size_t)T_pad * K * sizeof(_Float16);

@@ -204,6 +204,11 @@ struct IntForm {  // a projection's integer form: sub 32, 16 or 0 (none); min: a
 IntForm gemm_int_form(const MatvecSeg *seg, int n_seg);
 IntForm qkv_gemm_form(const flint_weight *wq, const flint_weight *wk, const flint_weight *wv);
 IntForm o_gemm_form(const flint_weight *wo);
+// whether a batch of n_tok tokens reads a projection's weight planes, kept by the caller or made for the call:
+// the integer form's short batches read the GGUF rows, and below GEMM_MIN_TOKENS there is no GEMM
+inline bool gemm_reads_planes(IntForm f, int n_tok, bool kept) {
+    return n_tok >= GEMM_MIN_TOKENS && !(f.sub && n_tok <= (kept ? GEMM_RAW_TOKENS_KEPT : GEMM_RAW_TOKENS));
+}
 size_t planes_bytes(int N, int K, IntForm f);
 WeightPlanes planes_at(void *mem, int N, int K, IntForm f);
 void build_qkv_planes(const flint_weight *wq, const flint_weight *wk, const flint_weight *wv, const WeightPlanes &pl,

@@ -160,8 +160,9 @@ struct flint_attn_model {
     int32_t n_ctx = 0, pos = 0;  // the session: context length and tokens processed
     // The prefill GEMMs' f16 hi/lo planes of every layer's q|k|v and o weights (75.5 MB a layer;
     // 40.1 MB in q8_0, whose GEMM keeps the integer values and the block scales), one allocation made at
-    // the first prefill block that takes the GEMM, layer il's at planes_off[il]; a layer's planes are built
-    // on the stream of its first such block and read by every later one. planes_on: the caller's
+    // the first prefill block with a projection that reads them (gemm_reads_planes), layer il's at
+    // planes_off[il]; a projection's planes are built (planes_built: 1 q|k|v, 2 o) on the stream of its first
+    // such block and read by every later one. planes_on: the caller's
     // switch (flint_attn_model_set_weight_planes). A failed allocation is tried once per prefill
     // call (planes_failed_call: the call it failed in), and the projections rebuild the planes in
     // the workspace meanwhile.
@@ -195,35 +196,43 @@ struct flint_attn_model {
     static size_t layer_planes_bytes(const Layer &L) {
         return qkv_planes_bytes(L) + planes_bytes(FLINT_N_EMBD, FLINT_Q_DIM, o_gemm_form(&L.o));
     }
-    // the layer's q|k|v and o planes, built on `stream` if this is the first use; false when
-    // there is no memory for them
-    bool layer_planes(int il, hipStream_t stream, WeightPlanes *pq_out, WeightPlanes *po_out) {
-        if (!planes_on) return false;
+    // the planes of the layer's projections that read them in a batch of n_tok tokens, built on `stream`
+    // if this is their first use: pq or po itself, null for a projection that reads none or without memory for them
+    struct LayerPlanes {
+        WeightPlanes q, o;
+        const WeightPlanes *pq = nullptr, *po = nullptr;
+    };
+    void layer_planes(int il, int n_tok, hipStream_t stream, LayerPlanes &P) {
+        const Layer &L = layers[il];
+        const IntForm fq = qkv_gemm_form(&L.q, &L.k, &L.v), fo = o_gemm_form(&L.o);
+        const bool want_q = gemm_reads_planes(fq, n_tok, true), want_o = gemm_reads_planes(fo, n_tok, true);
+        if (!planes_on || !(want_q || want_o)) return;
         if (!planes) {
-            if (planes_failed_call == prefill_call) return false;  // already failed in this call
+            if (planes_failed_call == prefill_call) return;  // already failed in this call
             planes_off.assign(layers.size() + 1, 0);
             for (size_t i = 0; i < layers.size(); i++) planes_off[i + 1] = planes_off[i] + layer_planes_bytes(layers[i]);
             if (hipMalloc(&planes, planes_off.back()) != hipSuccess) {
                 (void)hipGetLastError();  // clear the allocation error; the projections work without planes
                 planes = nullptr;
                 planes_failed_call = prefill_call;
-                return false;
+                return;
             }
             planes_failed_call = 0;
             planes_built.assign(layers.size(), 0);
         }
-        const Layer &L = layers[il];
         char *base = (char *)planes + planes_off[il];
-        const WeightPlanes pq = planes_at(base, FLINT_QKV_DIM, FLINT_N_EMBD, qkv_gemm_form(&L.q, &L.k, &L.v));
-        const WeightPlanes po = planes_at(base + qkv_planes_bytes(L), FLINT_N_EMBD, FLINT_Q_DIM, o_gemm_form(&L.o));
-        if (!planes_built[il]) {
-            build_qkv_planes(&L.q, &L.k, &L.v, pq, stream);
-            build_o_planes(&L.o, po, stream);
-            planes_built[il] = 1;
+        if (want_q) {
+            P.q = planes_at(base, FLINT_QKV_DIM, FLINT_N_EMBD, fq);
+            if (!(planes_built[il] & 1)) build_qkv_planes(&L.q, &L.k, &L.v, P.q, stream);
+            planes_built[il] |= 1;
+            P.pq = &P.q;
         }
-        *pq_out = pq;
-        *po_out = po;
-        return true;
+        if (want_o) {
+            P.o = planes_at(base + qkv_planes_bytes(L), FLINT_N_EMBD, FLINT_Q_DIM, fo);
+            if (!(planes_built[il] & 2)) build_o_planes(&L.o, P.o, stream);
+            planes_built[il] |= 2;
+            P.po = &P.o;
+        }
     }
     void reserve(int n_tok) {
         if (n_tok <= cap) return;
@@ -410,24 +419,13 @@ void block_prefill(flint_attn_model *m, int il, float *X, int p0, int T, float *
     float *a = att ? att : m->att;
     char e2[512] = {0};
     const hipStream_t s = (hipStream_t)stream;
-    WeightPlanes pq, po;
-    if (T >= GEMM_MIN_TOKENS && m->layer_planes(il, s, &pq, &po)) {
-        // the projections' GEMMs read the layer's cached weight planes
-        qkv_proj_rows_planes(&L.q, &L.k, &L.v, X, T, L.attn_norm, m->hp.h.rms_eps, m->qkv, FLINT_QKV_DIM, &pq, s);
-        m->stage(s, prof, il, "qkv");
-        call(flint_attn_engine_prefill(m->eng, il, m->qkv, p0, T, a, stream, e2, sizeof(e2)), e2);
-        m->stage(s, prof, il, "attn");
-        o_proj_rows_planes(&L.o, a, T, X, &po, s);
-        m->stage(s, prof, il, "o");
-        return;
-    }
-    call(flint_attn_qkv_proj_rows(&L.q, &L.k, &L.v, X, T, L.attn_norm, m->hp.h.rms_eps, m->qkv, FLINT_QKV_DIM,
-                                  stream, e2, sizeof(e2)),
-         e2);
+    flint_attn_model::LayerPlanes P;
+    m->layer_planes(il, T, s, P);
+    qkv_proj_rows_planes(&L.q, &L.k, &L.v, X, T, L.attn_norm, m->hp.h.rms_eps, m->qkv, FLINT_QKV_DIM, P.pq, s);
     m->stage(s, prof, il, "qkv");
     call(flint_attn_engine_prefill(m->eng, il, m->qkv, p0, T, a, stream, e2, sizeof(e2)), e2);
     m->stage(s, prof, il, "attn");
-    call(flint_attn_o_proj_rows(&L.o, a, T, X, stream, e2, sizeof(e2)), e2);
+    o_proj_rows_planes(&L.o, a, T, X, P.po, s);
     m->stage(s, prof, il, "o");
 }
 

@@ -167,28 +167,59 @@ def test_block_prefill_600_tokens(cuda, tmp_path):
     model.close()
 
 
-def test_weight_planes_switch(setup, cuda):
-    """The prefill projections' kept weight planes hold the bits the per-call weight prep writes:
-    prefill blocks with the planes kept, switched off (freed) and on again give bit-identical
-    hidden states, and the accessor reports each state."""
+@pytest.fixture(scope="module")
+def long_model(tmp_path_factory):
+    """The two-layer model with 600 positions, and the same with layer 1's o weights in f32 (no integer form)."""
+    m = mb.make_model(n_pos=600)
+    d = tmp_path_factory.mktemp("long")
+    paths = str(d / "int.gguf"), str(d / "f32.gguf")
+    mb.write_model(paths[0], m)
+    rows = np.random.default_rng(5).standard_normal((2048, 4096)).astype(np.float32) / 64
+    m["layers"][1]["o"] = ("f32", rows.view(np.uint8))
+    mb.write_model(paths[1], m)
+    return paths
+
+
+def _prefill_blocks(model, cuda, n):
+    """Hidden states of the model's first n tokens after both layers' prefill blocks, on the host."""
     import torch
-    path, embd, hidden, att, blocks = setup
-    n = embd.shape[0]
-    toks = list(range(n))
-    model = fa.Model(path, n_ctx=256)
+    X = torch.zeros((n, 2048), device=cuda)
+    model.embed(list(range(n)), X)
+    for il in range(2):
+        model.block_prefill(il, X, 0)
+    torch.cuda.synchronize()
+    return X.cpu().numpy()
+
+
+def test_weight_planes_switch(long_model, cuda):
+    """The prefill projections' kept weight planes hold the bits the per-call weight prep writes:
+    prefill blocks of 600 tokens (planes kept above 320 tokens, made for the call above 480) with the planes
+    kept, switched off (freed) and on again give bit-identical hidden states, and the accessor
+    reports each state."""
+    model = fa.Model(long_model[0], n_ctx=1024)
     assert model.weight_planes() == 2  # allowed, not allocated before the first prefill block
     outs = []
     for state in (1, 0, 1):
         model.set_weight_planes(state == 1)
-        X = torch.zeros((n, 2048), device=cuda)
-        model.embed(toks, X)
-        for il in range(2):
-            model.block_prefill(il, X, 0)
-        torch.cuda.synchronize()
+        outs.append(_prefill_blocks(model, cuda, 600))
         assert model.weight_planes() == state
-        outs.append(X.cpu().numpy())
     assert np.array_equal(outs[0], outs[1]) and np.array_equal(outs[0], outs[2])
-    _close(outs[0], hidden, "prefill hidden with kept planes, end to end")
+    model.close()
+
+
+@pytest.mark.parametrize("f32,sizes", [(False, ((320, 2), (321, 1), (320, 1), (481, 1))), (True, ((15, 2), (16, 1), (321, 1)))])
+def test_weight_planes_only_where_read(long_model, cuda, f32, sizes):
+    """A model allocates and builds its planes for the first block that reads them: above 320 tokens, or from 16
+    on where a projection has no integer form. On either side of the line, and at the sizes where a projection
+    without planes changes its own route (480 | 481 tokens), hidden states are the ones without planes."""
+    model = fa.Model(long_model[f32], n_ctx=1024)
+    for n, state in sizes:
+        kept = _prefill_blocks(model, cuda, n)
+        assert model.weight_planes() == state, n
+        off = fa.Model(long_model[f32], n_ctx=1024)
+        off.set_weight_planes(False)
+        assert np.array_equal(kept, _prefill_blocks(off, cuda, n)), n
+        off.close()
     model.close()
 
 
