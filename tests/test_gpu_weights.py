@@ -273,8 +273,9 @@ def _gemm_case(cuda, rng, types, wo_type, T, x_scale=None, att_scale=None):
 def test_projection_rows_gemm_matches_oracle(cuda, types, wo_type):
     """Batches from 16 tokens (the GEMM on f16 hi/lo planes, or on the weights' integer values
     and block scales for q8_0 / iq4_xs / q5_K / q6_K / f16 / bf16): every output within the fp32
-    reassociation bound of the oracle's double-accumulated matvec, at 131 tokens (a partial
-    128-token tile) in the engine's formats, the residual added in the o projection."""
+    reassociation bound of the oracle's double-accumulated matvec, at 131 tokens (a partial tile of the GEMM that
+    reads the GGUF rows, and of the hi/lo planes' where a weight is f32) in the engine's formats, the
+    residual added in the o projection."""
     _gemm_case(cuda, np.random.default_rng(51 + len(wo_type)), types, wo_type, 131)
 
 
@@ -290,7 +291,7 @@ def test_projection_rows_gemm_row_ranges(cuda):
 
 
 def test_projection_rows_gemm_1000_tokens(cuda):
-    """1000 tokens: eight 128-token tiles and a partial one, dealt over the XCDs tile by tile as a
+    """1000 tokens: fifteen 64-token tiles and a partial one, dealt over the XCDs tile by tile as a
     long prefill's are, every output within the bound of the oracle."""
     _gemm_case(cuda, np.random.default_rng(61), ("q8_0", "q6_K", "q5_K"), "q8_0", 1000)
 
@@ -320,6 +321,36 @@ def test_projection_rows_short_batches(cuda, types, wo_type):
         fa.qkv_proj_rows(*ws, x[a:].contiguous(), g, q_part[:n])
         y_part = torch.cat([x0[a:], x0[:1]])
         fa.o_proj_rows(wo, att[a:].contiguous(), y_part[:n])
+        torch.cuda.synchronize()
+        assert torch.equal(qkv[a:], q_part[:n]) and torch.isnan(q_part[n]).all(), ("qkv", types, n)
+        assert torch.equal(y[a:], y_part[:n]) and torch.equal(y_part[n], x0[0]), ("o", wo_type, n)
+
+
+@pytest.mark.parametrize("types,wo_type", [(("q8_0",) * 3, "q8_0"), (("q5_K",) * 3, "q5_K"), (("q5_K", "q8_0", "q6_K"), "q6_K"),
+                                           (("q6_K", "iq4_xs", "q6_K"), "iq4_xs"), (("iq4_xs",) * 3, "bf16"),
+                                           (("bf16", "f16", "q5_K"), "f16")])
+def test_projection_rows_long_batches(cuda, types, wo_type):
+    """Both tile sizes of the GEMM on weight planes where they meet and end raggedly: 1030 and 2048 tokens
+    (64-token tiles), 2049, 2100 and 2177 (128-token tiles; the last tile holds 1, 52 and 1 tokens), in every form
+    of the kernel (scales per 32 or 16 elements, with and without mins). Every row has the bits that the
+    short batches' GEMM, held against the oracle above, gives the same token; rows past the batch stay."""
+    import torch
+    rng = np.random.default_rng(73)
+    E, T = fa.N_EMBD, 2177
+    ws = [(_dev(oracle.random_blocks(t, n, E, rng), cuda), t) for t, n in zip(types, (4096, 512, 512))]
+    wo = (_dev(oracle.random_blocks(wo_type, E, 4096, rng), cuda), wo_type)
+    g = torch.rand(E, device=cuda) + 0.5
+    x, att, x0 = (torch.randn((T, n), device=cuda) for n in (E, 4096, E))
+    qkv, y = torch.empty((T, 5120), device=cuda), x0.clone()
+    for a in range(0, T, 311):  # 7 batches of 311 tokens
+        fa.qkv_proj_rows(*ws, x[a:a + 311], g, qkv[a:a + 311])
+        fa.o_proj_rows(wo, att[a:a + 311], y[a:a + 311])
+    for n in (1030, 2048, 2049, 2100, 2177):
+        a = T - n
+        q_part = torch.full((n + 1, 5120), float("nan"), device=cuda)
+        fa.qkv_proj_rows(*ws, x[a:], g, q_part[:n])
+        y_part = torch.cat([x0[a:], x0[:1]])
+        fa.o_proj_rows(wo, att[a:], y_part[:n])
         torch.cuda.synchronize()
         assert torch.equal(qkv[a:], q_part[:n]) and torch.isnan(q_part[n]).all(), ("qkv", types, n)
         assert torch.equal(y[a:], y_part[:n]) and torch.equal(y_part[n], x0[0]), ("o", wo_type, n)
