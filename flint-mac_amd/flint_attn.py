@@ -171,8 +171,12 @@ def _stream(stream):
     if stream is None:
         import torch
         # the handle of torch.cuda.current_stream() without its Stream object, which took 2.6 of the 7.6 us of a
-        # decode call (0.3 us this way); the device goes through current_device(), which initialises CUDA
-        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+        # decode call (0.3 us this way); the device goes through current_device(), which initialises CUDA.
+        # Not part of torch's public interface: without it, the Stream object
+        raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+        if raw is None:
+            return torch.cuda.current_stream().cuda_stream
+        return raw(torch.cuda.current_device())
     return stream
 
 

@@ -35,6 +35,17 @@ def test_probe_library_exports_its_entry_points():
     assert "flint_probe_" not in attn
 
 
+def test_current_stream_without_the_raw_handle(monkeypatch):
+    """The current stream's handle where torch lacks the private call that returns it directly: from the public one."""
+    import torch
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream", raising=False)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: type("S", (), {"cuda_stream": 1234})())
+    assert fa._stream(None) == 1234
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda device: 5678 + device, raising=False)
+    assert fa._stream(None) == 5678
+
+
 # The Rust server's bindings, as declared at /root/reference/server/src/ffi.rs:5-11 (the
 # #[repr(C)] config) and :19-29 (the extern "C" block), kept here as text.
 RUST_FFI = """
