@@ -482,6 +482,11 @@ constexpr int MT_MIN_TOKENS = 2;  // at 2 tokens matvec_tokens_kernel is ahead i
 int matvec_row_multiple(int k) { return MV_WAVES * (k == 2048 ? MV_ROWS_2048 : MV_ROWS_4096); }
 
 hipError_t launch_matvec(const MatvecParams &P, int k, hipStream_t stream) {
+    // a layer's two projections: matvec_kernel has the segments, the norm and the sum into y of each built in
+    const bool qkv = k == N_EMBD && P.n_seg == 3 && P.seg[1].row0 == Q_DIM && P.seg[2].row0 == Q_DIM + KV_DIM &&
+                     P.n_rows == QKV_DIM && P.norm_w && !P.add;
+    const bool o = k == Q_DIM && P.n_seg == 1 && P.n_rows == N_EMBD && !P.norm_w && P.add;
+    if (P.n_tok < 1 || P.seg[0].row0 != 0 || !(qkv || o)) return hipErrorInvalidValue;
     if (P.n_tok >= MT_MIN_TOKENS) {
         if (k == 2048) {
             constexpr int ROWS = MtShape<2048>::WAVES * MtShape<2048>::R;

@@ -35,6 +35,33 @@ def test_probe_library_exports_its_entry_points():
     assert "flint_probe_" not in attn
 
 
+class _Seg(ctypes.Structure):  # MatvecSeg of csrc/flint_attn_internal.h
+    _fields_ = [("w", ctypes.c_void_p), ("type", ctypes.c_int), ("row0", ctypes.c_int), ("row_bytes", ctypes.c_int)]
+
+
+class _Matvec(ctypes.Structure):  # MatvecParams
+    _fields_ = [("seg", _Seg * 3), ("n_seg", ctypes.c_int), ("n_rows", ctypes.c_int), ("x", ctypes.c_void_p),
+                ("norm_w", ctypes.c_void_p), ("eps", ctypes.c_float), ("y", ctypes.c_void_p), ("add", ctypes.c_int),
+                ("n_tok", ctypes.c_int), ("x_stride", ctypes.c_longlong), ("y_stride", ctypes.c_longlong)]
+
+
+@pytest.mark.parametrize("k,change", [(2048, {"norm_w": None}), (2048, {"add": 1}), (2048, {"n_seg": 1}), (2048, {"n_rows": 4096}),
+                                      (2048, {"n_tok": 0}), (4096, {"add": 0}), (4096, {"norm_w": 16}), (4096, {"n_rows": 5120}),
+                                      (1024, {})])
+def test_matvec_launch_refuses_what_its_kernel_has_not_built_in(k, change):
+    """The single-token matvec has the q|k|v and o projections' segments, norm and sum into y built in: parameters
+    that say otherwise are refused (hipErrorInvalidValue) before anything is launched, not dropped."""
+    launch = fa.lib()["_ZN5flint13launch_matvecERKNS_12MatvecParamsEiP12ihipStream_t"]
+    p = _Matvec(n_seg=3, n_rows=5120, x=16, norm_w=16, y=16, add=0, n_tok=1, x_stride=2048, y_stride=5120)
+    for i, row0 in enumerate((0, 4096, 4608)):
+        p.seg[i] = _Seg(16, 8, row0, 2176)
+    if k == 4096:
+        p.n_seg, p.n_rows, p.norm_w, p.add = 1, 2048, None, 1
+    for name, value in change.items():
+        setattr(p, name, value)
+    assert launch(ctypes.byref(p), ctypes.c_int(k), ctypes.c_void_p(0)) == 1
+
+
 def test_current_stream_without_the_raw_handle(monkeypatch):
     """The current stream's handle where torch lacks the private call that returns it directly: from the public one."""
     import torch
