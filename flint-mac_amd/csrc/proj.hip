@@ -314,17 +314,18 @@ __global__ __launch_bounds__(64 * MtShape<K>::WAVES) void matvec_tokens_kernel(c
     constexpr int UNITS = (QBYTES / 16 + 63) / 64;     // 16-byte loads per lane for it
     constexpr int QROW = (QBYTES + 4 + 15) / 16 * 16;  // a staged row, + 4 bytes read past a q8_0 row's end
     constexpr int XPT = K / 256;                       // x elements per thread: 256 threads a token, as matvec_kernel's
+    constexpr int N_ROWS = K == N_EMBD ? QKV_DIM : N_EMBD;
+    static_assert(N_ROWS % (WAVES * R) == 0 && KV_DIM % R == 0, "every workgroup is whole, a wave's rows in one segment");
     static_assert(SUBS * R == 2 && WAVES * R * QROW <= TOKENS * K * 4 && WAVES * 64 >= 512, "shape");
     __shared__ __align__(16) uint8_t lds[TOKENS * K * 4];  // the rows' bytes, then the x rows
     __shared__ double part[TOKENS][4];
     float *const xs = (float *)lds;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int row0 = (blockIdx.x * WAVES + wave) * R;  // R rows, all in one segment
-    const bool rows_ok = row0 < P.n_rows;              // the last workgroup's waves past the rows only stage x
     const MatvecSeg s0 = P.seg[0], s1 = P.seg[1], s2 = P.seg[2];
     const bool in2 = P.n_seg > 2 && row0 >= s2.row0, in1 = !in2 && P.n_seg > 1 && row0 >= s1.row0;
     const MatvecSeg S = in2 ? s2 : in1 ? s1 : s0;
-    const uint8_t *wrow = S.w + (size_t)((rows_ok ? row0 : S.row0) - S.row0) * S.row_bytes;
+    const uint8_t *wrow = S.w + (size_t)(row0 - S.row0) * S.row_bytes;
     const bool q8 = S.type == W_Q8_0;
     // this lane's weights: sub-block lane + 64 i of row r at w[r * SUBS + i] (q8_0: the quants, d their scale)
     float w[2][32], d[2] = {1.f, 1.f};
@@ -408,7 +409,7 @@ __global__ __launch_bounds__(64 * MtShape<K>::WAVES) void matvec_tokens_kernel(c
             }
         }
         // lane t: token t0 + t's row of y
-        const bool mine = lane < n && rows_ok;
+        const bool mine = lane < n;
         float *const y = P.y + (size_t)(t0 + (mine ? lane : 0)) * P.y_stride + row0;
         float yin[R], out[R];
 #pragma unroll
@@ -490,10 +491,10 @@ hipError_t launch_matvec(const MatvecParams &P, int k, hipStream_t stream) {
     if (P.n_tok >= MT_MIN_TOKENS) {
         if (k == 2048) {
             constexpr int ROWS = MtShape<2048>::WAVES * MtShape<2048>::R;
-            hipLaunchKernelGGL(matvec_tokens_kernel<2048>, dim3((P.n_rows + ROWS - 1) / ROWS), dim3(64 * MtShape<2048>::WAVES), 0, stream, P);
+            hipLaunchKernelGGL(matvec_tokens_kernel<2048>, dim3(P.n_rows / ROWS), dim3(64 * MtShape<2048>::WAVES), 0, stream, P);
         } else {
             constexpr int ROWS = MtShape<4096>::WAVES * MtShape<4096>::R;
-            hipLaunchKernelGGL(matvec_tokens_kernel<4096>, dim3((P.n_rows + ROWS - 1) / ROWS), dim3(64 * MtShape<4096>::WAVES), 0, stream, P);
+            hipLaunchKernelGGL(matvec_tokens_kernel<4096>, dim3(P.n_rows / ROWS), dim3(64 * MtShape<4096>::WAVES), 0, stream, P);
         }
         return hipGetLastError();
     }

@@ -941,7 +941,7 @@ static void launch_gemm_int(const GemmParams &G, hipStream_t stream) {
 // fetched whole lines for a quarter of their bytes and evicted each other's from the L1 (an unsegmented
 // form of this kernel at 512 tokens 121 us against 71 without those loads).
 
-constexpr int XPREP_FEW_ROWS = 512;  // see xprep_row_kernel
+static_assert(GEMM_RAW_TOKENS <= 512, "xprep_row_kernel is the faster one up to 512 rows");
 constexpr int GR_CHUNKS = GEMM_SEG / 32;    // chunks of a segment
 static_assert(GR_TILE == GEMM_RAW_TILE, "the x planes hold whole token tiles");
 
@@ -1101,10 +1101,7 @@ hipError_t launch_proj_gemm(const GemmWeightParams &W, const GemmActParams &X, c
     if (G.raw) {  // the integer form from the GGUF rows
         if (X.T_pad % GR_TILE != 0 || X.T_pad < G.T || G.T <= 0 || G.N % (8 * GR_TILE) != 0 || (G.isub != 32 && G.isub != 16))
             return hipErrorInvalidValue;
-        if (X.T_pad <= XPREP_FEW_ROWS)
-            hipLaunchKernelGGL(G.K == 2048 ? xprep_row_kernel<2048> : xprep_row_kernel<4096>, dim3(X.T_pad), dim3(G.K / 8), 0, stream, X);
-        else
-            hipLaunchKernelGGL(G.K == 2048 ? xprep_kernel<2048> : xprep_kernel<4096>, dim3(X.T_pad / 8), dim3(512), 0, stream, X);
+        hipLaunchKernelGGL(G.K == 2048 ? xprep_row_kernel<2048> : xprep_row_kernel<4096>, dim3(X.T_pad), dim3(G.K / 8), 0, stream, X);
         const int n_tt = X.T_pad / GR_TILE;
         void (*gk)(GemmParams, GemmWeightParams, int) =
             G.K == 2048 ? (G.isub == 32 ? gemm_raw_kernel<32, 2048 / GEMM_SEG> : gemm_raw_kernel<16, 2048 / GEMM_SEG>)
