@@ -330,8 +330,8 @@ def test_prefill_short_at_long_context_split_keys(cuda, store, is_swa):
     """Short prefills after a long one, where the prefill cuts every query block's key range
     into splits merged with the sink by a second kernel: continuations of T = 1, 7, 40, 100
     tokens from p0 = 20005 (full layer: 626-630 key tiles, 63 splits of 10 tiles for the
-    first three, 32 of 20 for T = 100) and from p0 = 5003 (SWA ring: at most 18 tiles, 3
-    splits of 6). Every new position against the oracle, at the usual bars."""
+    first two, 32 of 20 and 16 of 40) and from p0 = 5003 (SWA ring: at most 18 tiles, 9 splits of
+    2 for the first two, 5 of 4 and 3 of 6). Every new position against the oracle, at the usual bars."""
     p0 = 5003 if is_swa else 20005
     Ts = (1, 7, 40, 100)
     n = p0 + sum(Ts)
@@ -360,11 +360,12 @@ def test_prefill_short_at_long_context_split_keys(cuda, store, is_swa):
 
 
 @pytest.mark.parametrize("store", ["f16", "bf16"])
-@pytest.mark.parametrize("T,p0", [(1000, 0), (520, 33), (33, 63), (90, 991)])
+@pytest.mark.parametrize("T,p0", [(1000, 0), (520, 33), (33, 63), (90, 991), (1760, 230), (1376, 1600)])
 def test_prefill_blocks_whole_and_split(cuda, store, T, p0):
     """Causal calls whose shorter query blocks fit one key split and write their rows themselves while the
     longer ones are split and merged (1000 tokens: 16 whole blocks, 16 of two splits; ragged last
-    blocks), and calls whose blocks all have the same number of splits: every row against the oracle."""
+    blocks), calls whose blocks all have the same number of splits, and calls split for two rounds of
+    the CUs (1760 tokens: 2 splits of 32 tiles; 1376 at 1600: 3 of 31): every row against the oracle."""
     rng = np.random.default_rng(T + p0)
     qn, kn, sk = layer_weights(rng)
     n = p0 + T
