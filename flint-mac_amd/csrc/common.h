@@ -86,9 +86,6 @@ __host__ __device__ inline size_t vt_index(int kvh, int row, int dim, int rows) 
     return (((size_t)kvh * (rows >> 5) + (row >> 5)) * HEAD_DIM + dim) * 32 + (row & 31);
 }
 
-// Workgroup barrier that orders LDS only. __syncthreads() also orders global
-// memory, which the compiler implements by waiting for every outstanding global
-// load (s_waitcnt vmcnt(0)); this one leaves in-flight loads in flight.
 // Make the compiler materialise a wave-uniform value at this point: its scalar load is
 // issued here, together with the others pinned next to it, instead of being sunk to
 // its first use.
@@ -106,6 +103,9 @@ __device__ inline void wait_vmcnt() {  // s_waitcnt vmcnt(N), other counters unt
     __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
 }
 
+// Workgroup barrier that orders LDS only. __syncthreads() also orders global
+// memory, which the compiler implements by waiting for every outstanding global
+// load (s_waitcnt vmcnt(0)); this one leaves in-flight loads in flight.
 __device__ inline void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
     __builtin_amdgcn_s_barrier();

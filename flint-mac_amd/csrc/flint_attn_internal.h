@@ -168,15 +168,21 @@ struct GemmParams {
     int raw;               // the integer form straight from the GGUF rows (no weight planes)
 };
 constexpr int GEMM_RAW_TILE = 32;    // tokens and rows per gemm_raw workgroup
-// Batches of the integer form up to these sizes take gemm_raw. Stage-level calls, q/k/v + o in q8_0: 16, 128,
-// 256, 384, 448 and 512 tokens 26.7, 37.9, 59, 85, 103 and 112 us against 142-145 us for the weight planes'
-// build and 128-token tiles (99-110 us with 64-token tiles and the faster build): the lines cross at 480, since
-// gemm_raw's 32 x 32 tiles read x and the rows once each. With the planes kept (no build), 49 blocks: 256, 320 and 384
-// tokens 4.15, 5.12 and 5.53 ms against 5.10, 5.19 and 5.30.
+// Batches of the integer form up to these sizes take gemm_raw. Stage-level calls, q/k/v + o, us with gemm_raw | with
+// the weight planes' build and 64-token tiles at 384, 448, 480 and 512 tokens: q8_0 83 | 99, 101 | 108, 106 | 108,
+// 110 | 109; iq4_xs 86 | 100, 102 | 109, 108 | 109, 112 | 110; f16 83 | 101, 103 | 111, 108 | 111, 111 | 112; q6_K
+// 96 | 120, 115 | 129, 120 | 129, 124 | 130; q5_K 93 | 131, 113 | 140, 117 | 141, 120 | 141. The lines cross between 480
+// and 512 for q8_0 and iq4_xs and beyond 512 for the others (q5_K pays 20 us there for one line for all), since
+// gemm_raw's 32 x 32 tiles read x and the rows once each. With the planes kept (no build), 49 blocks in q8_0: 256,
+// 320 and 384 tokens 4.15, 5.12 and 5.53 ms against 5.10, 5.19 and 5.30.
 constexpr int GEMM_RAW_TOKENS = 480, GEMM_RAW_TOKENS_KEPT = 320;
 // Batches up to this size take gemm_int's 64-token tiles, whose smaller workgroups fill the GPU sooner and hold
-// four stages. q/k/v + o in q8_0 (trace medians): 600 tokens 39 + 48 us against 47 + 80 with 128-token tiles, 1024
-// 61 + 52 against 62 + 84, 2048 110 + 86 against 116 + 105; at 4000 the larger tile reads less: 194 + 152 us.
+// four stages. Stage-level calls, q/k/v + o, us with 64-token | with 128-token tiles: 1000 tokens q8_0 139 | 167, q5_K
+// 172 | 216, q6_K 159 | 183; 2048 222 | 233, 257 | 277, 239 | 245; 2100 275 | 267, 330 | 323, 306 | 290; 2400 278 | 272,
+// 333 | 328, 309 | 296; 3000 326 | 306, 388 | 368, 360 | 333; 4000 405 | 374, 491 | 445, 452 | 404 (iq4_xs and f16 as
+// q8_0). At 2048 tokens o is one whole round: the 512 workgroups of 64-token tiles that the GPU holds, or one of
+// 128-token tiles a CU. The next token starts another, so both step up, and from there the larger tile, which
+// reads less, is ahead.
 constexpr int GEMM_INT_64 = 2048;
 constexpr int GEMM_SEG = 512;         // the integer form sums K in segments of this many elements, then the segments
 constexpr int GEMM_TILE = 128;       // tokens and rows per gemm3 workgroup

@@ -291,9 +291,9 @@ __global__ __launch_bounds__(64 * MV_WAVES) void matvec_kernel(const uint8_t *w0
 // adding). Every sum has matvec_kernel's terms in its order, so a token has the single-token call's
 // bits. 256 workgroups of 10 (q/k/v) or 8 (o) waves: one round of the CUs; half the waves with twice the
 // rows each, which halves the LDS reads, measured slower (9 tokens 31 us, 15 tokens 39): too few waves to
-// cover the reads' latency. q/k/v + o, a workgroup a token -> here, of which 15.6 us is what two calls cost
-// the host: 9 tokens of q5_K 59.2 -> 24.3 us, of q8_0 35.1 -> 21.2, of bf16 62.3 -> 23.2; 15 tokens of q8_0
-// 52.7 -> 29.4; 2 tokens of q8_0 16.7 -> 15.9, of q5_K 18.4 -> 15.7; 2000 tokens into unaligned rows (q5_K o
+// cover the reads' latency. q/k/v + o, a workgroup a token -> here: 9 tokens of q5_K 59.2 -> 24.3 us, of q8_0
+// 35.1 -> 21.2, of bf16 62.3 -> 23.2; 15 tokens of q8_0 52.7 -> 29.4; 2 tokens (kernel times, trace medians) of
+// q8_0 7.5 + 6.3 -> 6.9 + 6.1, of q5_K 11.0 + 9.1 -> 8.8 + 7.5; 2000 tokens into unaligned rows (q5_K o
 // alone) 4817 -> 1281.
 template <int K>
 struct MtShape;
@@ -478,7 +478,7 @@ hipError_t launch_get_rows(const RowsParams &P, hipStream_t stream) {
 // 4096-element rows (o: 512 workgroups, two waves per SIMD: with one, each row's LDS reads and
 // FMA chain were exposed); measured best of 1, 2, 4 and 8 for either.
 constexpr int MV_ROWS_2048 = 2, MV_ROWS_4096 = 1;
-constexpr int MT_MIN_TOKENS = 2;  // at 2 tokens matvec_tokens_kernel is ahead in every type (q5_K 18.4 -> 15.7 us)
+constexpr int MT_MIN_TOKENS = 2;  // at 2 tokens matvec_tokens_kernel is ahead of a workgroup a token (figures above it)
 
 int matvec_row_multiple(int k) { return MV_WAVES * (k == 2048 ? MV_ROWS_2048 : MV_ROWS_4096); }
 

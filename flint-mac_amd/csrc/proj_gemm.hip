@@ -14,9 +14,10 @@
 //     the product) and scales each output by 2^(e_t + f_n), which is exact.
 // Three launches: wprep (weights -> planes), xprep (activations -> planes, the RMSNorm fused
 // for q/k/v) and gemm3 or gemm_int. The stage-level calls rebuild the weight planes from the GGUF
-// rows each time (~30 us for a layer's 19M weights); a model keeps every layer's planes after
+// rows each time (18-20 us for a layer's 19M weights in q8_0); a model keeps every layer's planes after
 // building them once, and its calls launch only xprep and the GEMM. Batches of up to
-// GEMM_RAW_TOKENS tokens in the integer form take gemm_raw instead, which reads the GGUF rows itself.
+// GEMM_RAW_TOKENS tokens (GEMM_RAW_TOKENS_KEPT with kept planes) in the integer form take gemm_raw instead,
+// which reads the GGUF rows itself.
 #include "common.h"
 #include "dequant.h"
 #include "flint_attn_internal.h"
@@ -159,7 +160,7 @@ __device__ inline uint2 lds8(const uint8_t *p, int odd) {
 // block j (a constant once unrolled), from its row in LDS: the values, the scales of elements
 // 0-15 and 16-31, and the min, in ggml's float order, so that scale * value - min is deq32's weight
 // (f16: scale 1; bf16: 8 significant bits, exact in f16 once the block's largest magnitude is scaled into
-// [2^14, 2^15): values below 2^-10 of it, beneath f16's normal range, round to f16's subnormal steps).
+// [2^14, 2^15): values below 2^-28 of it, beneath f16's normal range, round to f16's subnormal steps).
 template <int TYPE>
 struct RawRows;
 
@@ -699,8 +700,10 @@ __global__ __launch_bounds__(GM_THREADS, 2) void gemm3_kernel(const GemmParams P
 // segment each, gives the same bits; the segments' registers come from T in two half sets instead of
 // two whole ones.
 // What bounds it: at 4000 tokens (q8_0, trace medians) q/k/v 194 and o 152 us, 0.87 and 0.88 PF of MFMA
-// work; the matrix pipes are busy 44 % of the cycles, LDS indexed operations a quarter, and the rest
-// is waves waiting for each other at the chunk's barrier and for issue. (With whole T sets, no segments and
+// work; counters: the matrix pipes are busy 47-48 % of the launch's cycles (53-56 % of those in which a CU has
+// waves), LDS indexed operations 22 % without bank conflicts, and a wave spends 21 % of its time at waits
+// and barriers and 35 % ready but not issued. At 1000 tokens (64-token tiles) the pipes are busy 29 and
+// 26 %. (With whole T sets, no segments and
 // loads of 64-bit lane addresses: 195 and 158.)
 
 // 16 bytes a lane from base + voff (base wave-uniform) into LDS at dst + 16 lane. Inline asm: the builtin

@@ -143,8 +143,8 @@ def test_block_prefill_matches_oracle_and_decode(setup, cuda):
 
 def test_block_prefill_600_tokens(cuda, tmp_path):
     """A longer layer-major prefill (a model of the same layers with 600 positions): 600 tokens
-    through layer 0 and then layer 1 in one call each, so the projections run over five
-    128-token tiles and the flash kernel over 19 query blocks (and the 100-token window slides
+    through layer 0 and then layer 1 in one call each, so the projections run over ten
+    64-token tiles and the flash kernel over 19 query blocks (and the 100-token window slides
     over many). Each layer within the bars on its own input, and the hidden state end to end."""
     import torch
     m = mb.make_model(n_pos=600)
